@@ -30,6 +30,7 @@
 //     G * T of them per KV head, so each K/V page is still read once per KV
 //     head per 32 rows; token t sees keys j <= seq_len - T + t (the
 //     bottom-right causal convention of flashattn_tile/reference.py:19-22).
+#include <limits.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -70,20 +71,24 @@ __device__ __forceinline__ u32x4 kv_buffer_load(const uint8_t* base, int bytes, 
 #endif
 
 
-// Lane geometry for one 16-byte load per lane.
-template <int KV, int D>
+// Lane geometry: a row of D elements is held by at most 16 lanes, in kNc
+// 16-byte chunks each (chunk c + kLpr * j of lane c, so that a row's lanes
+// read consecutive chunks).
+template <typename QT, int KV, int D>
 struct Geom {
-  static constexpr int kElemBytes = (KV == KV_SAME) ? 2 : 1;
-  static constexpr int kEpl = 16 / kElemBytes;  // elements per lane per row
+  static constexpr int kElemBytes = (KV == KV_SAME) ? Elem<QT>::kBytes : 1;
+  static constexpr int kEpc = 16 / kElemBytes;  // elements per chunk
+  static constexpr int kNc = D / kEpc > 16 ? D / kEpc / 16 : 1;  // chunks per lane per row
+  static constexpr int kEpl = kEpc * kNc;       // elements per lane per row
   static constexpr int kLpr = D / kEpl;         // lanes per row
   static constexpr int kRpl = 64 / kLpr;        // rows per load
-  static constexpr int kNi16 = 16 / kRpl;       // loads per 16 tokens
-  // Tokens per streamed unit: 16, or 32 when 16 tokens take only two loads
-  // per lane for each of K and V (fp16/bf16 at head_dim 64), so a wave keeps
-  // as many bytes in flight as at head_dim 128.
-  static constexpr int kUnit = (KV == KV_SAME && kNi16 == 2) ? 32 : 16;
-  static constexpr int kUnitLog2 = kUnit == 32 ? 5 : 4;
-  static constexpr int kNi = kUnit / kRpl;      // loads per unit
+  static constexpr int kNi16 = kRpl < 16 ? 16 / kRpl : 1;  // row groups per 16 tokens
+  // Tokens per streamed unit: 16, or 32 or 64 when 16 tokens take only two
+  // or one loads per lane for each of K and V (fp16/bf16 at head_dim 64 or
+  // 32), so a wave keeps as many bytes in flight as at head_dim 128.
+  static constexpr int kUnitLog2 = (KV == KV_SAME && kNi16 == 2) ? 5 : (KV == KV_SAME && kNi16 == 1) ? 6 : 4;
+  static constexpr int kUnit = 1 << kUnitLog2;
+  static constexpr int kNi = kUnit / kRpl;      // row groups per unit
   static_assert(kLpr == 4 || kLpr == 8 || kLpr == 16, "unsupported head_dim / element size");
 };
 
@@ -112,10 +117,10 @@ __device__ __forceinline__ void transpose_reduce(float* x, int c) {
 }
 
 // Registers holding one unit's K/V rows (and per-load scales for 8-bit K/V).
-template <int NI>
+template <int NI, int NC>
 struct UnitRegs {
-  u32x4 k[NI];
-  u32x4 v[NI];
+  u32x4 k[NI * NC];
+  u32x4 v[NI * NC];
   float ksc[NI];
   float vsc[NI];
 };
@@ -344,16 +349,30 @@ __device__ __forceinline__ void merge_in_launch(const DecodeParams& p, int S, in
   if (threadIdx.x == 0) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename QT, int KV, int D, int HG, int NW>
+// LANE: K/V rows are addressed per lane (its own page id, a 64-bit address)
+// instead of per load, for pages that one load can straddle: page sizes below
+// RPL rows or not a power of two.  It also takes fp32 caches and head_dim 32
+// and 256, whatever the page size.  HBM-bound like the per-load form; a
+// lane's page ids are loaded one unit ahead of the rows they address (a
+// vector load, the 16 lanes of a row reading one word), so a unit's K/V loads
+// do not wait for them.  Against the LDS-tiled generic kernel that took these
+// shapes before (three workgroup barriers per 32 tokens), B32 with 32/8
+// heads: fp16 D128 page 1 ctx 2000 178 -> 46.5 us (5.65 TB/s), fp16 D256
+// page 16 ctx 1000 193 -> 45.8 us (5.7 TB/s), its int8 / fp8 205 -> 36.7 and
+// 202 -> 34.5 us, fp32 D128 page 16 ctx 1000 98 -> 43.3 us (6.1 TB/s).
+template <typename QT, int KV, int D, int HG, int NW, bool LANE = false>
 __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParams p) {
-  using Gm = Geom<KV, D>;
-  constexpr int EPL = Gm::kEpl, LPR = Gm::kLpr, RPL = Gm::kRpl, NI = Gm::kNi;
+  using Gm = Geom<QT, KV, D>;
+  constexpr int EPL = Gm::kEpl, LPR = Gm::kLpr, RPL = Gm::kRpl, NI = Gm::kNi, NC = Gm::kNc, EPC = Gm::kEpc;
+  constexpr bool F32Q = std::is_same<QT, F32>::value;
+  static_assert(LANE || (NC == 1 && !F32Q), "the per-load form takes one 16-bit or 8-bit chunk per lane");
   constexpr int NV = NI * HG;       // per-lane partial scores before the reduction
   constexpr int NPL = NV / LPR;     // scores per lane after it
   constexpr int VPH = NPL < NI ? NPL : NI;  // scores per lane per head
   constexpr int HPL = NPL / VPH;            // heads per lane
   constexpr int LPH = NI / VPH;             // lanes per head inside a row
-  constexpr int QW = EPL / 2;               // q dwords per head per lane (packed pairs)
+  constexpr int QW = F32Q ? EPL : EPL / 2;  // q dwords per head per lane (packed pairs, or fp32)
+  constexpr int QWC = QW / NC;              // of which per chunk
   static_assert(HG % 4 == 0, "HG must be a multiple of 4");
 
   __shared__ float s_p[NW][RPL][NV];
@@ -381,27 +400,63 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
   constexpr int UL = Gm::kUnitLog2;
   const int32_t* ptrow = p.pt + (int64_t)b * p.pt_sb;
   const bool early = split == 0 || p.pps_fixed > 0;
-  int first_pid[NI];
+  // LANE: this lane's page ids and slots of the unit that the next fetch
+  // reads.  Rows before `end` (INT_MAX: not clamped) look up their own token,
+  // later ones end - 1; table column and page id are clamped, so every
+  // address lies in the pool.
+  int lane_pid[NI], lane_slot[NI];
+  auto lookup = [&](int first_tok, int end) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const uint32_t tok = (uint32_t)min(first_tok + i * RPL + r, end - 1);
+      uint32_t lp;
+      if (p.log2P >= 0) {
+        lp = tok >> p.log2P;
+      } else {  // floor(tok / P): the high product is it or one less
+        lp = __umulhi(tok, p.invP);
+        lp += tok - lp * (uint32_t)p.P >= (uint32_t)p.P ? 1u : 0u;
+      }
+      lane_slot[i] = (int)(tok - lp * (uint32_t)p.P);
+      lane_pid[i] = ptrow[min((int)lp, p.max_pages - 1)];
+    }
+  };
   // Partition of this sequence's pages (decode.py:271-276 semantics).
-  int seq_len = first_page_ids<NI, RPL>(first_pid, ptrow, p, split, w << UL, b, early);
-  seq_len = max(0, min(seq_len, p.max_pages << p.log2P));
-  const int np = (seq_len + p.P - 1) >> p.log2P;
-  const int pps = p.pps_fixed > 0 ? p.pps_fixed : (np + S - 1) / S;
-  const int pb = split * pps;
-  const int pe = split == S - 1 ? np : min(np, pb + pps);
-  const int t_begin = pb << p.log2P;
-  const int t_end = min(seq_len, pe << p.log2P);
+  int first_pid[NI];
+  int t_begin, t_end;
+  if constexpr (LANE) {
+    // Fixed-size partitions and partition 0 begin at a page that does not
+    // depend on seq_len (a begin past the table is clamped by the lookup).
+    const int64_t cap = (int64_t)p.max_pages * p.P;
+    if (early) lookup((int)min((int64_t)split * p.pps_fixed * p.P, min(cap, (int64_t)1 << 30)) + (w << UL), INT_MAX);
+    const int seq_len = (int)max((int64_t)0, min((int64_t)p.lens[b], cap));
+    const int np = (int)(((int64_t)seq_len + p.P - 1) / p.P);
+    const int pps = p.pps_fixed > 0 ? p.pps_fixed : (np + S - 1) / S;
+    const int pb = (int)min((int64_t)np, (int64_t)split * pps);
+    const int pe = split == S - 1 ? np : (int)min((int64_t)np, (int64_t)pb + pps);
+    t_begin = pb * p.P;
+    t_end = (int)min((int64_t)seq_len, (int64_t)pe * p.P);
+  } else {
+    int seq_len = first_page_ids<NI, RPL>(first_pid, ptrow, p, split, w << UL, b, early);
+    seq_len = max(0, min(seq_len, p.max_pages << p.log2P));
+    const int np = (seq_len + p.P - 1) >> p.log2P;
+    const int pps = p.pps_fixed > 0 ? p.pps_fixed : (np + S - 1) / S;
+    const int pb = split * pps;
+    const int pe = split == S - 1 ? np : min(np, pb + pps);
+    t_begin = pb << p.log2P;
+    t_end = min(seq_len, pe << p.log2P);
+  }
   const int n_units = t_end > t_begin ? (t_end - t_begin + Gm::kUnit - 1) >> UL : 0;
 
-  // q for the HG heads, packed pairs of QT (padded heads reuse head0).
+  // q for the HG heads, packed pairs of QT or fp32 (padded heads reuse head0).
   u32 qv[HG][QW];
 #pragma unroll
   for (int g = 0; g < HG; ++g) {
     const int h = head0 + (g < nvalid ? g : 0);
-    const u32x4* qp = reinterpret_cast<const u32x4*>(p.q + 2 * (b * p.q_sb + h * p.q_sh + c * EPL));
 #pragma unroll
     for (int j = 0; j < QW / 4; ++j) {
-      const u32x4 t = qp[j];
+      // dword 4 j of the lane: chunk 4 j / QWC, 16 bytes 4 j % QWC / 4 of its q dwords
+      const int d = EPC * (c + LPR * (4 * j / QWC)) + (4 * j % QWC) * (F32Q ? 1 : 2);
+      const u32x4 t = *reinterpret_cast<const u32x4*>(p.q + Elem<QT>::kBytes * (b * p.q_sb + h * p.q_sh + d));
       qv[g][4 * j + 0] = t[0];
       qv[g][4 * j + 1] = t[1];
       qv[g][4 * j + 2] = t[2];
@@ -426,8 +481,34 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
   const uint32_t lane_v = r * vrow + EB * EPL * c;
 
   // first: u is this wave's first unit (first_pid holds its page ids).
-  auto fetch = [&](UnitRegs<NI>& R, int u, bool first) {
+  auto fetch = [&](UnitRegs<NI, NC>& R, int u, bool first) __attribute__((always_inline)) {
     const int base = t_begin + (u << UL);
+    if constexpr (LANE) {
+      int phys[NI], slot[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        phys[i] = min(max(lane_pid[i], 0), p.num_pages - 1);
+        slot[i] = lane_slot[i];
+      }
+      // The next unit's ids go out ahead of this unit's rows: loads return in
+      // order, so waiting for them leaves the rows in flight.
+      lookup(base + (NW << UL), t_end);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const uint8_t* kp = kh + ((uint64_t)(uint32_t)phys[i] * kpage + (uint64_t)(uint32_t)slot[i] * krow + 16 * c);
+        const uint8_t* vp = vh + ((uint64_t)(uint32_t)phys[i] * vpage + (uint64_t)(uint32_t)slot[i] * vrow + 16 * c);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+          R.k[i * NC + j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kp + 16 * LPR * j));
+          R.v[i * NC + j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vp + 16 * LPR * j));
+        }
+        if constexpr (KV != KV_SAME) {
+          R.ksc[i] = p.ks[(int64_t)phys[i] * p.sc_sp + (int64_t)kvh * p.sc_sh];
+          R.vsc[i] = p.vs[(int64_t)phys[i] * p.sc_sp + (int64_t)kvh * p.sc_sh];
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int rs = base + i * RPL;
@@ -468,8 +549,10 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = f[e] * sc;
       }
-      out[2 * j + 0] = Pair<QT>::pack(f[0], f[1]);
-      out[2 * j + 1] = Pair<QT>::pack(f[2], f[3]);
+      if constexpr (!F32Q) {
+        out[2 * j + 0] = Pair<QT>::pack(f[0], f[1]);
+        out[2 * j + 1] = Pair<QT>::pack(f[2], f[3]);
+      }
     }
   };
 
@@ -486,7 +569,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     for (int e = 0; e < EPL; ++e) acc[g][e] = 0.f;
 
   // One unit: scores, online softmax, PV.
-  auto process = [&](const UnitRegs<NI>& cur, int u) __attribute__((always_inline)) {
+  auto process = [&](const UnitRegs<NI, NC>& cur, int u) __attribute__((always_inline)) {
     const int base = t_begin + (u << UL);
 
     // ---- scores: partial q.k over this lane's EPL dims ----
@@ -494,19 +577,28 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       u32 kw[QW];
-      if constexpr (KV == KV_SAME) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) kw[j] = cur.k[i][j];
-      } else if constexpr (FOLD) {
-        k8_exact_f16<KV>(cur.k[i], kw);
-      } else {
-        deq_pairs(cur.k[i], cur.ksc[i], kw);
+      for (int n = 0; n < NC; ++n) {
+        if constexpr (KV == KV_SAME) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) kw[n * QWC + j] = cur.k[i * NC + n][j];
+        } else if constexpr (FOLD) {
+          u32 o[8];
+          k8_exact_f16<KV>(cur.k[i * NC + n], o);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) kw[n * QWC + j] = o[j];
+        } else {
+          deq_pairs(cur.k[i * NC + n], cur.ksc[i], &kw[n * QWC]);
+        }
       }
 #pragma unroll
       for (int g = 0; g < HG; ++g) {
         float s = 0.f;
 #pragma unroll
-        for (int j = 0; j < QW; ++j) s = Pair<QT>::dot2(qv[g][j], kw[j], s);
+        for (int j = 0; j < QW; ++j) {
+          if constexpr (F32Q) s = __builtin_fmaf(as_f32(qv[g][j]), as_f32(kw[j]), s);
+          else s = Pair<QT>::dot2(qv[g][j], kw[j], s);
+        }
         part[g * NI + i] = FOLD ? s * cur.ksc[i] : s;  // load i's rows share one page
       }
     }
@@ -594,16 +686,23 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     for (int i = 0; i < NI; ++i) {
       float vf[EPL];
       u32 vw[QW];
-      if constexpr (KV == KV_SAME) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) vw[j] = cur.v[i][j];
-      } else {
-        deq_pairs(cur.v[i], cur.vsc[i], vw);
+      for (int n = 0; n < NC; ++n) {
+        if constexpr (KV == KV_SAME) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) vw[n * QWC + j] = cur.v[i * NC + n][j];
+        } else {
+          deq_pairs(cur.v[i * NC + n], cur.vsc[i], &vw[n * QWC]);
+        }
       }
 #pragma unroll
       for (int j = 0; j < QW; ++j) {
-        vf[2 * j] = Pair<QT>::lo(vw[j]);
-        vf[2 * j + 1] = Pair<QT>::hi(vw[j]);
+        if constexpr (F32Q) {
+          vf[j] = as_f32(vw[j]);
+        } else {
+          vf[2 * j] = Pair<QT>::lo(vw[j]);
+          vf[2 * j + 1] = Pair<QT>::hi(vw[j]);
+        }
       }
 #pragma unroll
       for (int g = 0; g < HG; ++g) {
@@ -616,11 +715,28 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
 
   // Two register sets, unit u + NW loading while unit u is processed (the
   // loop is unrolled by two so that no copy moves one set into the other).
-  UnitRegs<NI> nxt;
+  UnitRegs<NI, NC> nxt;
+  if constexpr (LANE) {
+    if (!early && w < n_units) lookup(t_begin + (w << UL), t_end);
+  }
   if (w < n_units) fetch(nxt, w, true);
   for (int u = w; u < n_units; u += NW) {
-    const UnitRegs<NI> cur = nxt;
+    UnitRegs<NI, NC> cur = nxt;
     if (u + NW < n_units) fetch(nxt, u + NW, false);
+    if constexpr (LANE) {
+      // Rows past t_end hold other tokens' data: their scores are masked,
+      // and zero V rows keep p * v = 0 (the per-load form reads zeros there).
+      if (t_begin + ((u + 1) << UL) > t_end) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const bool in = t_begin + (u << UL) + i * RPL + r < t_end;
+#pragma unroll
+          for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cur.v[i * NC + n][j] = in ? cur.v[i * NC + n][j] : 0u;
+        }
+      }
+    }
     process(cur, u);
   }
 
@@ -638,7 +754,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
 #pragma unroll
     for (int g = 0; g < HG; ++g)
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) s_red[w][g][c * EPL + e] = acc[g][e];
+      for (int e = 0; e < EPL; ++e) s_red[w][g][(c + LPR * (e / EPC)) * EPC + e % EPC] = acc[g][e];
 #pragma unroll
     for (int hh = 0; hh < HPL; ++hh) {
       const int j0 = c * NPL + hh * VPH;
@@ -668,9 +784,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     }
     const int h = head0 + g;
     if (S == 1) {
-      const float o = L > 0.f ? A / L : 0.f;
-      uint16_t* op = reinterpret_cast<uint16_t*>(p.out) + (b * p.o_sb + h * p.o_sh + d);
-      *op = Pair<QT>::from_float(o);
+      store_elem<QT>(p.out, b * p.o_sb + h * p.o_sh + d, L > 0.f ? A / L : 0.f);
     } else {
       const int64_t row = ((int64_t)b * p.H + h) * S + split;
       const bool coh = p.counters != nullptr;
@@ -1106,6 +1220,52 @@ int launch_decode_q(const fat::DecodeParams& prm, int kv, int D, int HG, int nw,
 }
 
 
+// Per-lane addressing (paged_decode_kernel<..., LANE>), 4-head groups.
+template <typename QT, int KV, int D>
+int launch_lane_t(const fat::DecodeParams& prm, int nw, dim3 grid, hipStream_t stream) {
+  if (nw == 8) {
+    hipLaunchKernelGGL((fat::paged_decode_kernel<QT, KV, D, 4, 8, true>), grid, dim3(8 * 64), 0, stream, prm);
+  } else {
+    hipLaunchKernelGGL((fat::paged_decode_kernel<QT, KV, D, 4, 4, true>), grid, dim3(4 * 64), 0, stream, prm);
+  }
+  return fat_host::launch_status("paged_decode_kernel");
+}
+
+// The shapes it is built for: at least four lanes per row (fp16/bf16 and fp32
+// from head_dim 32, 8-bit from 64) and a unit's registers without spills
+// (head_dim up to 256, fp32 up to 128).
+bool lane_takes(int q_dtype, int kv, int D) {
+  const int lo = kv == fat::KV_SAME ? 32 : 64;
+  return D >= lo && D <= (q_dtype == FAT_DTYPE_F32 ? 128 : 256);
+}
+
+template <typename QT, int KV>
+int launch_lane_kv(const fat::DecodeParams& prm, int D, int nw, dim3 grid, hipStream_t stream) {
+  if constexpr (KV == fat::KV_SAME) {
+    if (D == 32) return launch_lane_t<QT, KV, 32>(prm, nw, grid, stream);
+  }
+  if constexpr (!std::is_same<QT, fat::F32>::value) {
+    if (D == 256) return launch_lane_t<QT, KV, 256>(prm, nw, grid, stream);
+  }
+  return D == 128 ? launch_lane_t<QT, KV, 128>(prm, nw, grid, stream)
+                  : launch_lane_t<QT, KV, 64>(prm, nw, grid, stream);
+}
+
+template <typename QT>
+int launch_lane_q(const fat::DecodeParams& prm, int kv, int D, int nw, dim3 grid, hipStream_t stream) {
+  switch (kv) {
+    case fat::KV_SAME: return launch_lane_kv<QT, fat::KV_SAME>(prm, D, nw, grid, stream);
+    case fat::KV_I8: return launch_lane_kv<QT, fat::KV_I8>(prm, D, nw, grid, stream);
+    default: return launch_lane_kv<QT, fat::KV_FP8>(prm, D, nw, grid, stream);
+  }
+}
+
+int launch_lane(const fat::DecodeParams& prm, int q_dtype, int kv, int D, int nw, dim3 grid, hipStream_t stream) {
+  if (q_dtype == FAT_DTYPE_F16) return launch_lane_q<fat::F16>(prm, kv, D, nw, grid, stream);
+  if (q_dtype == FAT_DTYPE_BF16) return launch_lane_q<fat::BF16>(prm, kv, D, nw, grid, stream);
+  return launch_lane_kv<fat::F32, fat::KV_SAME>(prm, D, nw, grid, stream);
+}
+
 template <typename QT, int KV, int NW>
 void launch_decode_mfma_kvw(const fat::DecodeParams& prm, int D, dim3 grid, hipStream_t stream) {
   if (D == 128)
@@ -1294,6 +1454,15 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   }
 
   const int group = a->num_heads / a->num_kv_heads;
+  // Of the shapes the fast kernels refuse, the VALU kernel's per-lane form
+  // takes those it is built for, with 16-byte aligned queries and strides
+  // that fit its 32-bit factors; the generic kernel keeps the rest.  A group
+  // of more than 4 heads reads its K/V once per 4 heads, most of it from L2,
+  // and is still the faster form (fp16 page 1, B32: 64/8 heads ctx 2000 223 ->
+  // 90.6 us, 32/1 heads ctx 8000 262 -> 101 us; fp32 64/8 ctx 1000 123 -> 82.6).
+  const uintptr_t lane_align = (uintptr_t)a->q | (uintptr_t)(qeb * a->q_stride_b) | (uintptr_t)(qeb * a->q_stride_h);
+  const bool lane = generic && a->kernel == FAT_KERNEL_AUTO && lane_takes(a->q_dtype, kv, D) &&
+                    strides_ok && (lane_align & 15) == 0;
   bool use_mfma = group >= fat::kDecMfmaMinGroup || (kv != fat::KV_SAME && FAT_DEC_MFMA_8BIT);
   if (a->kernel == FAT_KERNEL_DECODE_VALU || a->kernel == FAT_KERNEL_DECODE_MFMA)
     use_mfma = a->kernel == FAT_KERNEL_DECODE_MFMA;
@@ -1303,7 +1472,8 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
                         "(group %d); use FAT_KERNEL_AUTO or FAT_KERNEL_DECODE_MFMA", group);
     return FAT_E_UNSUPPORTED;
   }
-  const int HG = generic ? (group < fat_host::kGenericHeads ? group : fat_host::kGenericHeads)
+  const int HG = lane ? 4
+                 : generic ? (group < fat_host::kGenericHeads ? group : fat_host::kGenericHeads)
                          : (use_mfma ? 32 : (group >= 8 ? 8 : 4));
   const int hg_per_kv = (group * T + HG - 1) / HG;
 
@@ -1341,6 +1511,7 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   prm.hg_per_kv = hg_per_kv;
   prm.P = a->page_size;
   prm.log2P = log2P;
+  prm.invP = a->page_size > 1 ? (uint32_t)((uint64_t(1) << 32) / (uint32_t)a->page_size) : 0;
   prm.num_pages = a->num_pages;
   prm.max_pages = a->max_pages;
   prm.pps_fixed = a->pages_per_split;
@@ -1365,6 +1536,15 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
   const int64_t pages_per_wg =
       a->pages_per_split > 0 ? a->pages_per_split : ((int64_t)a->max_pages + a->split_k - 1) / a->split_k;
+  if (lane) {
+    const int nw = a->waves_per_group ? a->waves_per_group
+                                      : ((wgs < 2 * 256 || pages_per_wg * a->page_size >= 1024) ? 8 : 4);
+    fused = use_fused(std::min(HG, group), nw);
+    prm.counters = fused ? a->merge_counters : nullptr;
+    const int rc = launch_lane(prm, a->q_dtype, kv, D, nw, grid, stream);
+    if (rc != FAT_OK || a->split_k == 1 || fused) return rc;
+    return launch_merge(prm, a, D, stream);
+  }
   if (generic) {
     const int rc = fat_host::launch_decode_generic(prm, a->q_dtype, kv, D, HG, grid, stream);
     if (rc != FAT_OK || a->split_k == 1) return rc;

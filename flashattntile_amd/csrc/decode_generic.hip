@@ -1,7 +1,7 @@
 // decode_generic.hip -- paged decode for the shapes the VALU and MFMA decode
-// kernels (decode.hip) do not take: fp32 queries and caches, page sizes that
-// are not a power of two or are below the rows one 16-byte load per lane
-// covers, and head_dim 16, 32, 256 or 512.
+// kernels (decode.hip) do not take: head_dim 16 and 512, fp32 at head_dim
+// 256, 8-bit caches at head_dim 32, queries whose rows are not 16-byte
+// aligned, and K/V strides beyond the other kernels' 32-bit factors.
 //
 // Semantics are those of the other decode kernels and of the reference's
 // native decode (csrc/paged_decode.cu:80-235): one query per sequence, query

@@ -31,6 +31,7 @@ struct DecodeParams {
   int32_t H, Hkv, group, hg_per_kv;
   int32_t T;  // query tokens per sequence (1 = single-query decode)
   int32_t P, log2P, num_pages, max_pages;  // log2P = -1: page_size not a power of two
+  uint32_t invP;  // floor(2^32 / page_size), page_size > 1
   int32_t pps_fixed;  // pages per partition, 0 = ceil(np / split_k)
   float scale_log2;  // softmax_scale * log2(e)
   // Split-K merge inside the decode launch: one counter per (sequence, head

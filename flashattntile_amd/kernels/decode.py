@@ -57,9 +57,9 @@ __all__ = [
 # but the HIP kernel's pipeline depth is fixed (one 16-token unit prefetched
 # per wave).  kernel None lets the library choose the kernel family; "valu",
 # "mfma" or "generic" forces one (what a tuning run stores for its shape; the
-# generic kernel is the library's own choice only for the shapes the other
-# two do not take: fp32, page sizes below their floor or not a power of two,
-# head_dim 32 or 256).
+# generic kernel is the library's own choice only for the shapes the VALU
+# kernel's per-lane form does not take either: head_dim 16 and 512, fp32 at
+# head_dim 256, 8-bit caches at head_dim 32, unaligned queries).
 DEFAULT_CONFIG = {"split_k": None, "num_warps": None, "num_stages": 2, "pages_per_split": None, "kernel": None}
 
 _KERNEL_CODES = {None: _hip.KERNEL_AUTO, "valu": _hip.KERNEL_DECODE_VALU, "mfma": _hip.KERNEL_DECODE_MFMA,

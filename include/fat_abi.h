@@ -131,9 +131,11 @@ enum fat_status {
  * ids are clamped to [0, num_pages)).  The VALU and MFMA kernels take
  * fp16/bf16 queries, head_dim 64 or 128 and power-of-two pages of at least
  * the rows one 16-byte load per lane covers: 4 (fp16/bf16, head_dim 128), 8
- * (fp16/bf16 64; int8/fp8 128) or 16 (int8/fp8 64).  Every other request
- * runs on the generic kernel (one query per sequence only); fp32 queries
- * take an fp32 cache.
+ * (fp16/bf16 64; int8/fp8 128) or 16 (int8/fp8 64).  FAT_KERNEL_AUTO runs
+ * other page sizes, fp32 caches (to head_dim 128) and head_dim 32 and 256 on
+ * the VALU kernel's per-lane form and every other request on the generic
+ * kernel (one query per sequence only on both); fp32 queries take an fp32
+ * cache.
  *   out      [batch, num_heads, head_dim]          q_dtype
  * Strides are in elements; the head_dim axis must be contiguous.
  *
