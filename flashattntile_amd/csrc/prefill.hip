@@ -1253,8 +1253,9 @@ bool valid_prefill_kernel(int kernel) {
          kernel == FAT_KERNEL_PREFILL_GENERIC;
 }
 
-// fp32 and head_dim 16 / 512 have no MFMA prefill kernel: the generic one
-// (prefill_generic.hip) takes them; forcing it runs it on any shape.
+// fp32 and head_dim 16 / 512 take no fp16/bf16 MFMA kernel: the generic one
+// (prefill_generic.hip) or, for packed fp32 at head_dim 32-128, the fp32 one
+// (prefill_f32.hip) does; forcing the generic kernel runs it on any shape.
 bool prefill_needs_generic(int dtype, int D) { return dtype == FAT_DTYPE_F32 || D == 16 || D == 512; }
 
 // Whether the bf16 V pre-pass can run for a packed launch (its arrays fit
@@ -1352,6 +1353,10 @@ int launch_prefill(fat::PrefillParams& prm, int max_seqlen_q, int64_t max_seqlen
       fat_host::set_error("%s: too many query blocks (%lld)", who, (long long)n);
       return FAT_E_UNSUPPORTED;
     }
+    // Packed fp32 at head_dim 32-128 runs on the fp32 matrix instructions;
+    // paged fp32, other head dims and a forced generic kernel stay there.
+    if (PG == 0 && dtype == FAT_DTYPE_F32 && D >= 32 && D <= 128 && kernel == FAT_KERNEL_AUTO)
+      return fat_host::launch_prefill_f32(prm, D, causal, dim3((unsigned)n), stream);
     return fat_host::launch_prefill_generic(prm, dtype, D, causal, PG != 0, dim3((unsigned)n), stream);
   }
   const bool vpre_ok = PG == 0 && workspace && vpre_fits(prm.B, prm.Hkv, D, total_k, max_seqlen_k);

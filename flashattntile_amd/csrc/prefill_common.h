@@ -1,5 +1,5 @@
-// prefill_common.h -- what the prefill kernels of prefill.hip and
-// prefill_wide.hip share: the launch parameters, the tile constants, the
+// prefill_common.h -- what the prefill kernels of prefill.hip,
+// prefill_wide.hip and prefill_f32.hip share: the launch parameters, the tile constants, the
 // lazy-rescale bounds of the ping-pong kernels and the epilogue that writes
 // a wave's output rows through LDS.
 #pragma once
@@ -99,6 +99,24 @@ __device__ __forceinline__ void write_rows_via_lds(uint16_t* ob, int li, int g, 
   }
 }
 
+typedef __attribute__((address_space(3))) void lds_void;
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes per lane from buffer `desc` at byte offset `voff` straight into
+// LDS at `lds_addr` + 16 * lane (lds_addr wave-uniform, in M0).  Offsets past
+// the descriptor's range arrive as zeros.  An SALU write of M0 needs one wait
+// state before a load that writes LDS (the s_nop).  Nothing else in the
+// kernels keeps a value in M0.
+__device__ __forceinline__ void buffer_load_lds16(const i32x4& desc, int voff, int lds_addr) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %1, 0 offen lds"
+      :
+      : "v"(voff), "s"(desc), "s"(lds_addr)
+      : "memory", "m0");
+}
+
 }  // namespace fat
 
 namespace fat_host {
@@ -112,6 +130,9 @@ int launch_prefill_wide(const fat::PrefillParams& prm, bool bf16, bool causal, d
 // query rows.
 int launch_prefill_generic(const fat::PrefillParams& prm, int dtype, int D, bool causal, bool paged, dim3 grid,
                            hipStream_t stream);
+// The packed fp32 prefill on fp32 MFMAs (prefill_f32.hip), head_dim 32, 64 or
+// 128; `grid` counts blocks of 32 query rows.
+int launch_prefill_f32(const fat::PrefillParams& prm, int D, bool causal, dim3 grid, hipStream_t stream);
 // Packed copies of a paged launch's K/V rows (prefill_stage.hip): cu_k
 // [B + 1] from `paged`.lens clamped to `cap`, then every sequence's rows into
 // kdst / vdst as [cu_k[B], Hkv, D] (2-byte elements, head_dim 128).

@@ -1,6 +1,7 @@
 // prefill_generic.hip -- varlen prefill for the shapes the MFMA prefill
-// kernels (prefill.hip, prefill_wide.hip) do not take: fp32 inputs, and
-// head_dim 16 or 512 (every power of two from 16 to 512 runs here when forced).
+// kernels (prefill.hip, prefill_wide.hip, prefill_f32.hip) do not take: paged
+// fp32, fp32 at head_dim 256, and head_dim 16 or 512 (every power of two from
+// 16 to 512 runs here when forced).
 //
 // Semantics are those of the other prefill kernels and of the reference's
 // _fwd_varlen_kernel (flashattn_tile/kernels/prefill.py:35-138): per (query

@@ -86,24 +86,6 @@ struct WideOrder {
 #define FAT_WIDE_LOOK 2
 #endif
 
-typedef __attribute__((address_space(3))) void lds_void;
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// 16 bytes per lane from buffer `desc` at byte offset `voff` straight into
-// LDS at `lds_addr` + 16 * lane (lds_addr wave-uniform, in M0).  Offsets past
-// the descriptor's range arrive as zeros.  An SALU write of M0 needs one wait
-// state before a load that writes LDS (the s_nop).  Nothing else in the
-// kernel keeps a value in M0.
-__device__ __forceinline__ void buffer_load_lds16(const i32x4& desc, int voff, int lds_addr) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %0, %1, 0 offen lds"
-      :
-      : "v"(voff), "s"(desc), "s"(lds_addr)
-      : "memory", "m0");
-}
-
 // Longest-first order of a packed launch's work items.  Item i = (query
 // block jb = i / B counted from the sequence's end, sequence b = i % B); its
 // causal chain holds kv_len - 512 jb keys (kv_len when not causal).  Items

@@ -14,9 +14,10 @@ waves, 128 rows, the two 4-wave groups taking alternate key tiles),
 ``config=None`` the stored winner for the shape is used
 (:func:`flashattntile_amd.autotune.best_config`, the reference's lookup at
 ``prefill.py:167-191``).  There is no CPU fallback: non-ROCm tensors raise.
-fp32 inputs, and head_dim 16 or 512, always run on ``"generic"`` (the
-reference sends fp32 to its fp32 torch path, ``prefill.py:286-290``);
-forcing ``"generic"`` runs it on any shape.
+Packed fp32 inputs at head_dim 32 to 128 run on an fp32 matrix kernel of
+their own (``kernel`` None; the reference sends fp32 to its fp32 torch path,
+``prefill.py:286-290``), other fp32 inputs and head_dim 16 or 512 on
+``"generic"``; forcing ``"generic"`` runs it on any shape.
 
 ``paged_prefill_attention`` is the paged (chunked) form the reference lacks:
 the queries of each sequence attend to that sequence's keys in a

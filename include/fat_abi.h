@@ -219,7 +219,8 @@ typedef struct fat_decode_args {
  *   non-decreasing, kv_len >= q_len per sequence when causal.
  *   out [total_q, num_heads, head_dim]      dtype
  * dtype is fp16, bf16 or fp32; head_dim a power of two from 16 to 512.
- * fp32 and head_dim 16 / 512 run on the generic kernel only
+ * fp32 and head_dim 16 / 512 run on the generic kernel (AUTO: packed fp32 at
+ * head_dim 32 to 128 on an fp32 matrix kernel)
  * (FAT_KERNEL_AUTO or FAT_KERNEL_PREFILL_GENERIC); head_dim 256 at fp16 /
  * bf16 on the 4-wave kernel (or the generic one); a kernel that does not
  * take the shape returns FAT_E_UNSUPPORTED.  The same holds for
