@@ -14,13 +14,14 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libfat_hip.so"
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 # enum fat_dtype
 DT_F16 = 0
@@ -60,6 +61,8 @@ EXPORTED_SYMBOLS = (
     "fat_quantize_pages",
     "fat_append_kv",
     "fat_cache_stats",
+    "fat_check_begin",
+    "fat_check_wait",
 )
 
 _c_i64 = ctypes.c_int64
@@ -271,6 +274,36 @@ class CacheStatsArgs(ctypes.Structure):
     ]
 
 
+# enum fat_check_kind
+CHECK_CACHE = 0
+CHECK_VARLEN = 1
+CHECK_PAGED = 2
+CHECK_APPEND = 3
+CHECK_RANGE = 4
+CHECK_RESULTS = 16
+CHECK_HOST_WORDS = CHECK_RESULTS + 2 * 64
+
+
+class CheckArgs(ctypes.Structure):
+    """Mirror of ``fat_check_args``."""
+
+    _fields_ = [
+        ("cu_q", _c_vp),
+        ("cu_k", _c_vp),
+        ("seq_lens", _c_vp),
+        ("page_table", _c_vp),
+        ("page_table_stride", _c_i64),
+        ("host", _c_vp),
+        ("ticket", _c_i64),
+        ("kind", _c_i32),
+        ("batch", _c_i32),
+        ("max_pages", _c_i32),
+        ("page_size", _c_i32),
+        ("values", _c_vp),
+        ("count", _c_i64),
+    ]
+
+
 _LOCK = threading.Lock()
 _LIB: ctypes.CDLL | None = None
 _ERROR: str | None = None
@@ -322,11 +355,17 @@ def _load() -> None:
         lib.fat_append_kv.argtypes = [ctypes.POINTER(AppendArgs), _c_vp]
         lib.fat_cache_stats.restype = ctypes.c_int
         lib.fat_cache_stats.argtypes = [ctypes.POINTER(CacheStatsArgs), _c_vp]
+        lib.fat_check_begin.restype = ctypes.c_int
+        lib.fat_check_begin.argtypes = [ctypes.POINTER(CheckArgs), _c_vp]
+        lib.fat_check_wait.restype = ctypes.c_int
+        lib.fat_check_wait.argtypes = [ctypes.POINTER(CheckArgs), _c_vp, _c_vp]
         _LIB = lib
 
 
 def is_loaded() -> bool:
     """Load the library once; True if it is usable."""
+    if _LIB is not None:
+        return True
     _load()
     return _LIB is not None
 
@@ -339,33 +378,125 @@ def load_error() -> str:
 
 def lib() -> ctypes.CDLL:
     """The loaded library; raises RuntimeError (no fallback) when unavailable."""
+    if _LIB is not None:
+        return _LIB
     _load()
     if _LIB is None:
         raise RuntimeError(f"HIP kernel library unavailable: {_ERROR}")
     return _LIB
 
 
+class Check:
+    """The device-side checks of one validated call (``fat_check_begin`` /
+    ``fat_check_wait``): begun when constructed by :func:`check_begin`, and
+    waited for by :meth:`wait`; the caller prepares its launch in between.
+
+    One per (thread, device), reused: it holds the page-locked words that the
+    kernel writes.  A check that was begun and never waited for (an exception
+    in between) is drained before its words are used again."""
+
+    def __init__(self, device: torch.device) -> None:
+        with torch.cuda.device(device):
+            self._host = torch.zeros(CHECK_HOST_WORDS, dtype=torch.int64, pin_memory=True)
+        self._device = device
+        self._args = CheckArgs()
+        self._args.host = self._host.data_ptr()
+        self._ref = ctypes.byref(self._args)
+        self._result = (_c_i64 * CHECK_RESULTS)()
+        self._ticket = 0
+        self._stream = 0
+        self._pending = False
+
+    def begin(self, kind: int, batch: int, stream: int, cu_q: torch.Tensor | None, cu_k: torch.Tensor | None,
+              seq_lens: torch.Tensor | None, page_table: torch.Tensor | None, page_size: int) -> None:
+        if self._pending:
+            torch.cuda.synchronize(self._device)
+        a = self._args
+        a.kind = kind
+        a.batch = batch
+        a.cu_q = None if cu_q is None else cu_q.data_ptr()
+        a.cu_k = None if cu_k is None else cu_k.data_ptr()
+        if seq_lens is not None:
+            a.seq_lens = seq_lens.data_ptr()
+            a.page_table = page_table.data_ptr()
+            a.page_table_stride = page_table.stride(0)
+            a.max_pages = page_table.shape[1]
+            a.page_size = page_size
+        self._ticket += 1
+        a.ticket = self._ticket
+        self._stream = stream
+        self._pending = True
+        rc = lib().fat_check_begin(self._ref, stream)
+        if rc != 0:
+            self._pending = False
+            _check(rc, "fat_check_begin")
+
+    def begin_range(self, values: torch.Tensor, stream: int) -> None:
+        if self._pending:
+            torch.cuda.synchronize(self._device)
+        a = self._args
+        a.kind = CHECK_RANGE
+        a.values = values.data_ptr()
+        a.count = values.numel()
+        self._ticket += 1
+        a.ticket = self._ticket
+        self._stream = stream
+        self._pending = True
+        rc = lib().fat_check_begin(self._ref, stream)
+        if rc != 0:
+            self._pending = False
+            _check(rc, "fat_check_begin")
+
+    def wait(self) -> list[int]:
+        """The results (``fat_check_wait``), once the GPU has written them."""
+        _check(lib().fat_check_wait(self._ref, self._stream, self._result), "fat_check_wait")
+        self._pending = False
+        return list(self._result)
+
+
+_CHECKS = threading.local()
+
+
+def _thread_check(device: torch.device) -> Check:
+    checks = _CHECKS.__dict__
+    check = checks.get(device.index)
+    if check is None:
+        check = checks[device.index] = Check(device)
+    return check
+
+
+def float_range(values: torch.Tensor) -> tuple[float, float]:
+    """Min and max of a non-empty contiguous fp32 ROCm tensor (NaN if it
+    holds one, as torch's), one launch and one poll."""
+    check = _thread_check(values.device)
+    check.begin_range(values, current_stream_handle(values.device))
+    r = check.wait()
+    lo, hi = struct.unpack("ff", struct.pack("ii", r[12], r[13]))
+    return lo, hi
+
+
+def check_begin(kind: int, stream: int, device: torch.device, cu_q: torch.Tensor | None = None,
+                cu_k: torch.Tensor | None = None, seq_lens: torch.Tensor | None = None,
+                page_table: torch.Tensor | None = None, page_size: int = 0) -> Check:
+    """Begin a check on ``stream``: ``cu_q`` / ``cu_k`` int32 [B + 1],
+    ``seq_lens`` int32 [B] (contiguous), ``page_table`` int32 [B, M > 0] with
+    a unit column stride, B > 0, on one ROCm device."""
+    check = _thread_check(device)
+    batch = seq_lens.shape[0] if seq_lens is not None else cu_q.shape[0] - 1
+    check.begin(kind, batch, stream, cu_q, cu_k, seq_lens, page_table, page_size)
+    return check
+
+
 def cache_stats(seq_lens: torch.Tensor, page_table: torch.Tensor, page_size: int) -> list[int]:
-    """``fat_cache_stats`` on the current stream, then one copy back:
-    ``[min_len, max_len, min_page, max_page, total_pages]`` (the page range
-    over the columns the longest sequence uses; INT32_MAX / INT32_MIN when
-    none).  ``seq_lens`` int32 [B] contiguous, ``page_table`` int32 [B, M]
-    with a contiguous last axis."""
-    out = torch.empty(5, dtype=torch.int64, device=seq_lens.device)
-    a = CacheStatsArgs()
-    a.seq_lens = _ptr(seq_lens)
-    a.page_table = _ptr(page_table)
-    a.page_table_stride = page_table.stride(0)
-    a.batch = seq_lens.shape[0]
-    a.max_pages = page_table.shape[1]
-    a.page_size = int(page_size)
-    a.out = _ptr(out)
-    stream = torch.cuda.current_stream(seq_lens.device)
-    _check(lib().fat_cache_stats(ctypes.byref(a), _c_vp(int(stream.cuda_stream))), "fat_cache_stats")
-    host = torch.empty(5, dtype=torch.int64, pin_memory=True)
-    host.copy_(out, non_blocking=True)
-    stream.synchronize()
-    return host.tolist()
+    """``[min_len, max_len, min_page, max_page, total_pages]`` of a paged
+    cache (the page range over the columns the longest sequence uses;
+    INT32_MAX / INT32_MIN when none), one launch and one poll.  ``seq_lens``
+    int32 [B] contiguous, ``page_table`` int32 [B, M] with a contiguous last
+    axis, B and M positive."""
+    dev = seq_lens.device
+    r = check_begin(CHECK_CACHE, current_stream_handle(dev), dev, seq_lens=seq_lens, page_table=page_table,
+                    page_size=int(page_size)).wait()
+    return [r[0], r[1], r[12], r[13], r[2]]
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -389,7 +520,9 @@ def _check(rc: int, what: str) -> None:
 
 
 def current_stream_handle(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    # torch's raw handle of the current stream, without a Stream object
+    index = device.index
+    return int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index))
 
 
 def decode_workspace_bytes(batch: int, num_heads: int, head_dim: int, split_k: int) -> int:

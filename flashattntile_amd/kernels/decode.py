@@ -69,6 +69,8 @@ _KERNEL_CODES = {None: _hip.KERNEL_AUTO, "valu": _hip.KERNEL_DECODE_VALU, "mfma"
 # type); int8 / float8_e4m3fn caches take fp16 / bf16 queries.
 _DECODE_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
+_NO_PAGE = torch.iinfo(torch.int32).max  # the check's page range when no column is used
+
 _QUANT_DTYPES = tuple(d for d in (torch.int8, getattr(torch, "float8_e4m3fn", None)) if d is not None)
 
 
@@ -147,12 +149,15 @@ def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: i
     return resolved
 
 
-def _validate_decode_inputs(q: torch.Tensor, cache: PagedKVCache, multi: bool = False) -> tuple[int, int]:
-    """``decode.py:503-522`` + ``paging.validate_cache``, with one sync.
+def _validate_decode_inputs(q: torch.Tensor, cache: PagedKVCache, multi: bool = False,
+                            prepare=None) -> tuple[int, int, tuple | None]:
+    """``decode.py:503-522`` + ``paging.validate_cache``, with one host wait.
 
     ``multi``: ``q`` is ``[batch, q_len, heads, head_dim]`` and every sequence
-    must already hold its q_len new tokens.  Returns ``(max_len,
-    total_pages)`` for the partition heuristic."""
+    must already hold its q_len new tokens.  ``prepare``: called while the
+    check kernel of ROCm tensors runs (its errors are left to the caller's
+    own checks).  Returns ``(max_len, total_pages)`` for the partition
+    heuristic and what ``prepare`` returned (None: not called, or it raised)."""
     if not isinstance(cache, PagedKVCache):
         raise TypeError("cache must be a PagedKVCache")
     _check_layout(cache)
@@ -171,7 +176,22 @@ def _validate_decode_inputs(q: torch.Tensor, cache: PagedKVCache, multi: bool = 
         raise ValueError("q and cache must live on the same device")
     if not q.is_floating_point():
         raise ValueError(f"q must be floating point, got {q.dtype}")
-    min_len, max_len, lo, hi, total_pages = cache_stats(cache, with_total_pages=True)
+    sl, pt = cache.seq_lens, cache.page_table
+    prepared = None
+    if prepare is not None and sl.is_cuda and sl.is_contiguous() and pt.stride(-1) == 1 and pt.numel() \
+            and _hip.is_loaded():
+        check = _hip.check_begin(_hip.CHECK_CACHE, _hip.current_stream_handle(sl.device), sl.device, seq_lens=sl,
+                                 page_table=pt, page_size=cache.page_size)
+        try:
+            prepared = prepare()
+        except Exception:
+            prepared = None
+        r = check.wait()
+        min_len, max_len, lo, hi, total_pages = r[0], r[1], r[12], r[13], r[2]
+        if lo == _NO_PAGE:
+            lo, hi = 0, -1
+    else:
+        min_len, max_len, lo, hi, total_pages = cache_stats(cache, with_total_pages=True)
     if min_len < 0:
         raise AssertionError("seq_lens must be non-negative")
     capacity = cache.capacity
@@ -187,7 +207,7 @@ def _validate_decode_inputs(q: torch.Tensor, cache: PagedKVCache, multi: bool = 
     if multi and min_len < q.shape[1]:
         raise ValueError(f"multi-token decode requires every sequence to hold its {q.shape[1]} new tokens "
                          f"(shortest seq_len {min_len})")
-    return max_len, total_pages
+    return max_len, total_pages, prepared
 
 
 def _require_rocm(q: torch.Tensor, cache: PagedKVCache, what: str) -> None:
@@ -214,8 +234,8 @@ def merge_counters(q: torch.Tensor, split_k: int) -> torch.Tensor | None:
         return None
     rows = q.shape[0] * (q.shape[1] if q.dim() == 4 else 1)
     n = rows * q.shape[-2]  # fat_paged_decode_counters_bytes / 4: one int32 per (query row, head)
-    key = (q.device.index if q.device.index is not None else torch.cuda.current_device(),
-           _hip.current_stream_handle(q.device))
+    dev = q.device
+    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _hip.current_stream_handle(dev))
     t = _MERGE_COUNTERS.get(key)
     if t is None or t.numel() < n:
         t = torch.zeros(max(n, 4096), dtype=torch.int32, device=q.device)
@@ -247,6 +267,16 @@ def paged_decode_launch(
     only this stream's launches use); the decode launch then merges its
     partitions itself.  None: a second kernel merges.
     """
+    a, out, _keep = _decode_block(q, cache, softmax_scale, scales, out)
+    _launch_block(a, q, split_k, workspace=workspace, waves_per_group=waves_per_group,
+                  pages_per_split=pages_per_split, kernel=kernel, counters=counters)
+    return out
+
+
+def _decode_block(q, cache, softmax_scale, scales=None, out=None):
+    """The argument block of a decode launch but for its partitions
+    (:func:`_launch_block`), its output, and the tensors that have to live
+    until the launch is enqueued."""
     if cache.k_cache.stride(-1) != 1 or cache.v_cache.stride(-1) != 1:
         raise ValueError("k_cache and v_cache need a contiguous head_dim axis")
     if out is None:
@@ -255,22 +285,56 @@ def paged_decode_launch(
     # densely (the reference honours any strides, kernels/decode.py:89).
     pt = cache.page_table if cache.page_table.stride(-1) == 1 else cache.page_table.contiguous()
     sl = cache.seq_lens if cache.seq_lens.is_contiguous() else cache.seq_lens.contiguous()
-    rows = q.shape[0] * (q.shape[1] if q.dim() == 4 else 1)
-    need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], split_k)
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     k_scale = v_scale = None
     if scales is not None:
         k_scale = scales["k"] if isinstance(scales, dict) else scales.k
         v_scale = scales["v"] if isinstance(scales, dict) else scales.v
+    a = _hip.decode_args(q, cache.k_cache, cache.v_cache, pt, sl, out, cache.page_size, softmax_scale, 1,
+                         k_scale=k_scale, v_scale=v_scale)
+    return a, out, (q, pt, sl, k_scale, v_scale)
+
+
+def _launch_block(a, q, split_k, workspace=None, waves_per_group=None, pages_per_split=0, kernel=None,
+                  counters=None) -> None:
+    """Enqueue the block of :func:`_decode_block` with these partitions."""
+    rows = q.shape[0] * (q.shape[1] if q.dim() == 4 else 1)
+    need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], split_k) if split_k > 1 else 0
+    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     # fat_paged_decode_counters_bytes: one int32 per (query row, head)
     if counters is not None and counters.numel() * counters.element_size() < 4 * rows * q.shape[-2]:
         raise ValueError("paged_decode_launch: counters smaller than decode_counters_bytes(rows, num_heads)")
-    _hip.paged_decode(q, cache.k_cache, cache.v_cache, pt, sl, out,
-                      cache.page_size, softmax_scale, split_k, workspace=workspace,
-                      k_scale=k_scale, v_scale=v_scale, waves_per_group=waves_per_group or 0,
-                      pages_per_split=pages_per_split, kernel=_KERNEL_CODES[kernel], counters=counters)
+    a.split_k = int(split_k)
+    a.workspace = None if workspace is None else workspace.data_ptr()
+    a.waves_per_group = waves_per_group or 0
+    a.pages_per_split = int(pages_per_split)
+    a.kernel = _KERNEL_CODES[kernel]
+    a.merge_counters = None if counters is None else counters.data_ptr()
+    _hip.decode_with_args(a, _hip.current_stream_handle(q.device))
+
+
+def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
+    """Launch with the resolved partitions, from the prepared block if there
+    is one."""
+    q = q.contiguous()
+    if prepared is None:
+        prepared = _decode_block(q, cache, scale, scales)
+    a, out, keep = prepared
+    _launch_block(a, q, cfg["split_k"], waves_per_group=cfg["num_warps"], pages_per_split=cfg["pages_per_split"],
+                  kernel=cfg["kernel"], counters=merge_counters(q, cfg["split_k"]))
+    del keep
     return out
+
+
+def _dense_scales(scales) -> dict:
+    """``{"k", "v"}`` of QuantScales or such a dict, contiguous."""
+    k_scale = scales["k"] if isinstance(scales, dict) else scales.k
+    v_scale = scales["v"] if isinstance(scales, dict) else scales.v
+    return {"k": k_scale.contiguous(), "v": v_scale.contiguous()}
+
+
+def _scale_of(q, softmax_scale) -> float:
+    return float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
 
 
 def paged_decode_attention(
@@ -292,18 +356,16 @@ def paged_decode_attention(
     ``q.dtype``.
     """
     del grouped  # every launch is grouped on MI355X
-    max_len, total_pages = _validate_decode_inputs(q, cache)
-    scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
+    max_len, total_pages, prepared = _validate_decode_inputs(
+        q, cache, prepare=lambda: _decode_block(q.contiguous(), cache, _scale_of(q, softmax_scale)))
+    scale = _scale_of(q, softmax_scale)
     cfg = _resolve_config(config, q, cache, max_len, total_pages)
     _require_rocm(q, cache, "paged_decode_attention")
     if q.dtype not in _DECODE_DTYPES:
         raise ValueError(f"paged_decode_attention: dtype {q.dtype} is not fp16/bf16/fp32 (the HIP kernels' types)")
     if cache.k_cache.dtype != q.dtype:
         raise ValueError(f"q dtype {q.dtype} must match cache dtype {cache.k_cache.dtype}")
-    q = q.contiguous()
-    return paged_decode_launch(q, cache, scale, cfg["split_k"], waves_per_group=cfg["num_warps"],
-                               pages_per_split=cfg["pages_per_split"], kernel=cfg["kernel"],
-                               counters=merge_counters(q, cfg["split_k"]))
+    return _decode(q, cache, scale, cfg, prepared)
 
 
 def paged_decode_attention_fp8(
@@ -319,7 +381,9 @@ def paged_decode_attention_fp8(
     with ``"k"``/``"v"``), fp32 ``[num_pages, num_kv_heads]``.  Pages are
     dequantised in registers as ``(float(x) * scale).to(q.dtype)``.
     """
-    max_len, total_pages = _validate_decode_inputs(q, cache)
+    max_len, total_pages, prepared = _validate_decode_inputs(
+        q, cache, prepare=lambda: _decode_block(q.contiguous(), cache, _scale_of(q, softmax_scale),
+                                                _dense_scales(scales)))
     k_scale = scales["k"] if isinstance(scales, dict) else scales.k
     v_scale = scales["v"] if isinstance(scales, dict) else scales.v
     quant_dtype = cache.k_cache.dtype
@@ -328,7 +392,7 @@ def paged_decode_attention_fp8(
     expected = (cache.num_pages, cache.num_kv_heads)
     if tuple(k_scale.shape) != expected or tuple(v_scale.shape) != expected:
         raise ValueError(f"scales must have shape {expected}, got {tuple(k_scale.shape)}")
-    scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
+    scale = _scale_of(q, softmax_scale)
     cfg = _resolve_config(config, q, cache, max_len, total_pages)
     _require_rocm(q, cache, "paged_decode_attention_fp8")
     if not (k_scale.is_cuda and v_scale.is_cuda):
@@ -337,11 +401,7 @@ def paged_decode_attention_fp8(
         raise ValueError(f"quantised decode requires fp16/bf16 queries, got {q.dtype}")
     if k_scale.dtype != torch.float32 or v_scale.dtype != torch.float32:
         raise ValueError("scales must be float32")
-    q = q.contiguous()
-    return paged_decode_launch(q, cache, scale, cfg["split_k"],
-                               scales={"k": k_scale.contiguous(), "v": v_scale.contiguous()},
-                               waves_per_group=cfg["num_warps"], pages_per_split=cfg["pages_per_split"],
-                               kernel=cfg["kernel"], counters=merge_counters(q, cfg["split_k"]))
+    return _decode(q, cache, scale, cfg, prepared, _dense_scales(scales) if prepared is None else None)
 
 
 def paged_decode_attention_multi(
@@ -361,14 +421,16 @@ def paged_decode_attention_multi(
     ``{"k", "v"}``) selects an int8/float8_e4m3fn cache.  ``config`` as for
     :func:`paged_decode_attention`.  Returns ``q``'s shape and dtype.
     """
-    max_len, total_pages = _validate_decode_inputs(q, cache, multi=True)
+    max_len, total_pages, prepared = _validate_decode_inputs(
+        q, cache, multi=True, prepare=lambda: _decode_block(q.contiguous(), cache, _scale_of(q, softmax_scale),
+                                                            None if scales is None else _dense_scales(scales)))
     q_len = int(q.shape[1])
     if q_len > 64:
         raise ValueError(f"multi-token decode takes at most 64 tokens per sequence, got {q_len}")
     quantized = cache.k_cache.dtype in _QUANT_DTYPES
     if quantized != (scales is not None):
         raise ValueError("an int8/float8 cache needs scales, and only such a cache takes them")
-    scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
+    scale = _scale_of(q, softmax_scale)
     cfg = _resolve_config(config, q, cache, max_len, total_pages, q_len=q_len)
     _require_rocm(q, cache, "paged_decode_attention_multi")
     if q.dtype not in (torch.float16, torch.bfloat16):
@@ -382,13 +444,10 @@ def paged_decode_attention_multi(
             raise ValueError(f"scales must have shape {expected}, got {tuple(k_scale.shape)}")
         if k_scale.dtype != torch.float32 or v_scale.dtype != torch.float32:
             raise ValueError("scales must be float32")
-        sc = {"k": k_scale.contiguous(), "v": v_scale.contiguous()}
+        sc = _dense_scales(scales) if prepared is None else None
     elif cache.k_cache.dtype != q.dtype:
         raise ValueError(f"q dtype {q.dtype} must match cache dtype {cache.k_cache.dtype}")
-    q = q.contiguous()
-    return paged_decode_launch(q, cache, scale, cfg["split_k"], scales=sc,
-                               waves_per_group=cfg["num_warps"], pages_per_split=cfg["pages_per_split"],
-                               kernel=cfg["kernel"], counters=merge_counters(q, cfg["split_k"]))
+    return _decode(q, cache, scale, cfg, prepared, sc)
 
 
 class DecodeLaunch:
@@ -414,7 +473,7 @@ class DecodeLaunch:
                  total_pages: int | None = None) -> None:
         multi = q.dim() == 4
         if max_len is None or total_pages is None:
-            max_len, total_pages = _validate_decode_inputs(q, cache, multi=multi)
+            max_len, total_pages, _ = _validate_decode_inputs(q, cache, multi=multi)
         q_len = int(q.shape[1]) if multi else 1
         cfg = _resolve_config(config, q, cache, max_len, total_pages, q_len=q_len)
         _require_rocm(q, cache, "DecodeLaunch")

@@ -81,10 +81,8 @@ def _resolve_config(config: dict | None, kind: str | None = None, signature: str
     return resolved
 
 
-def _validate_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k, causal) -> tuple[int, int]:
-    """``prefill.py:194-233`` with the device-side checks in one sync.
-
-    Returns the longest query and key sequence lengths."""
+def _check_shapes(q, k, v, cu_seqlens_q, cu_seqlens_k) -> None:
+    """The host-only checks of ``prefill.py:194-233``."""
     if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
         raise ValueError("q, k, v must be 3-D [tokens, heads, head_dim]")
     if k.shape != v.shape:
@@ -107,6 +105,11 @@ def _validate_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k, causal) -> tuple[int, 
         raise ValueError("cu_seqlens_q and cu_seqlens_k must be int32")
     if cu_seqlens_q.device != q.device or cu_seqlens_k.device != q.device:
         raise ValueError("cu_seqlens must live on the same device as q")
+
+
+def _varlen_stats(cu_seqlens_q, cu_seqlens_k) -> list[int]:
+    """What ``_judge_varlen`` checks, by torch reductions and one copy (CPU
+    tensors; ROCm tensors take the check kernel)."""
     cq = cu_seqlens_q.to(torch.int64)
     ck = cu_seqlens_k.to(torch.int64)
     lq = cq[1:] - cq[:-1]
@@ -119,7 +122,14 @@ def _validate_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k, causal) -> tuple[int, 
         (lk < lq).any().to(torch.int64), lq.max(), lk.max(),
         keyless.any().to(torch.int64), first_keyless, lq[first_keyless],
     ]).cpu().tolist()
-    q0, k0, q_end, k_end, q_dec, k_dec, short_kv, max_q, max_k, any_keyless, kl_b, kl_q = (int(x) for x in stats)
+    return [int(x) for x in stats]
+
+
+def _judge_varlen(stats, q, k, causal) -> tuple[int, int]:
+    """The device-side checks of ``prefill.py:194-233`` on their numbers.
+
+    Returns the longest query and key sequence lengths."""
+    q0, k0, q_end, k_end, q_dec, k_dec, short_kv, max_q, max_k, any_keyless, kl_b, kl_q = stats
     if q0 != 0 or k0 != 0:
         raise ValueError("cu_seqlens must start at 0")
     if q_end != q.shape[0]:
@@ -159,6 +169,16 @@ def prefill_launch(
     must bound every sequence (they size the launch grid).  ``kernel``:
     None (library's choice), ``"pingpong"``, ``"wide"``, ``"4wave"``, ``"4wave_split"`` or ``"generic"``.
     """
+    a, out, _keep = _prefill_block(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal,
+                                   softmax_scale, out, workspace, kernel)
+    _hip.prefill_varlen_with_args(a, _hip.current_stream_handle(q.device))
+    return out
+
+
+def _prefill_block(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, softmax_scale, out=None,
+                   workspace=None, kernel=None):
+    """The argument block of :func:`prefill_launch`, its output, and the
+    tensors that have to live until the launch is enqueued."""
     if q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1:
         raise ValueError("q, k, v need a contiguous head_dim axis")
     if out is None:
@@ -176,8 +196,7 @@ def prefill_launch(
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace = workspace.data_ptr()
-    _hip.prefill_varlen_with_args(a, _hip.current_stream_handle(q.device))
-    return out
+    return a, out, (q, k, v, cu_seqlens_q, cu_seqlens_k, workspace)
 
 
 def prefill_attention(
@@ -199,8 +218,25 @@ def prefill_attention(
     on the same ROCm device; causal masking is bottom-right aligned.  Returns
     ``[total_q, num_heads, head_dim]`` in ``q.dtype``.
     """
-    longest_q, longest_k = _validate_inputs(q, k, v, cu_seqlens_q, cu_seqlens_k, causal)
-    scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
+    _check_shapes(q, k, v, cu_seqlens_q, cu_seqlens_k)
+    # ROCm tensors: the check kernel runs while the launch is prepared.  An
+    # error of the preparation is raised after those of the validation.
+    check = block = error = None
+    if q.is_cuda and _hip.is_loaded():
+        stream = _hip.current_stream_handle(q.device)
+        cq = cu_seqlens_q if cu_seqlens_q.is_contiguous() else cu_seqlens_q.contiguous()
+        ck = cu_seqlens_k if cu_seqlens_k.is_contiguous() else cu_seqlens_k.contiguous()
+        check = _hip.check_begin(_hip.CHECK_VARLEN, stream, q.device, cu_q=cq, cu_k=ck)
+        try:
+            block = _prepare(q, k, v, cq, ck, max_seqlen_q, max_seqlen_k, causal, softmax_scale, config)
+        except Exception as exc:
+            error = exc
+        r = check.wait()
+        flags, first = r[7], r[10]
+        stats = [r[3], r[5], r[4], r[6], flags & 1, flags & 2, flags & 4, r[8], r[9], first >= 0, first, r[11]]
+    else:
+        stats = _varlen_stats(cu_seqlens_q, cu_seqlens_k)
+    longest_q, longest_k = _judge_varlen(stats, q, k, causal)
     if max_seqlen_q <= 0:
         raise ValueError(f"max_seqlen_q must be positive, got {max_seqlen_q}")
     if max_seqlen_k <= 0:
@@ -211,10 +247,25 @@ def prefill_attention(
         raise ValueError(f"max_seqlen_q {max_seqlen_q} is smaller than the longest query sequence {longest_q}")
     if max_seqlen_k < longest_k:
         raise ValueError(f"max_seqlen_k {max_seqlen_k} is smaller than the longest key sequence {longest_k}")
+    if error is not None:
+        raise error
+    if block is None:  # not ROCm tensors (or no library): the preparation names what is missing
+        block = _prepare(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, softmax_scale,
+                         config)
+        stream = _hip.current_stream_handle(q.device)
+    a, out, _keep = block
+    _hip.prefill_varlen_with_args(a, stream)
+    return out
+
+
+def _prepare(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, softmax_scale, config):
+    """What :func:`prefill_attention` does besides the validation and the
+    launch: the launch's argument block, its output, and what it refers to."""
+    scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
     sig = prefill_signature(cu_seqlens_q.shape[0] - 1, q.shape[1], k.shape[1], q.shape[2], int(max_seqlen_q),
                             int(max_seqlen_k), causal)
     cfg = _resolve_config(config, "prefill", sig)
-    if not all(t.is_cuda for t in (q, k, v, cu_seqlens_q, cu_seqlens_k)):
+    if not (q.is_cuda and k.is_cuda and v.is_cuda and cu_seqlens_q.is_cuda and cu_seqlens_k.is_cuda):
         raise RuntimeError("prefill_attention: inputs must be ROCm device tensors; this build runs the gfx950 "
                            "HIP kernel only (no CPU or reference fallback)")
     if q.dtype not in _PREFILL_DTYPES:
@@ -222,16 +273,13 @@ def prefill_attention(
     q = q if q.stride(-1) == 1 else q.contiguous()
     k = k if k.stride(-1) == 1 else k.contiguous()
     v = v if v.stride(-1) == 1 else v.contiguous()
-    return prefill_launch(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), int(max_seqlen_k),
-                          bool(causal), scale, kernel=cfg["kernel"])
+    return _prefill_block(q, k, v, cu_seqlens_q, cu_seqlens_k, int(max_seqlen_q), int(max_seqlen_k), bool(causal),
+                          scale, kernel=cfg["kernel"])
 
 
-def _validate_paged(q, cache: PagedKVCache, cu_seqlens_q, causal) -> int:
-    """Shape/dtype checks plus the device-side ones (cu_seqlens_q monotone
-    and ending at q.shape[0]; lengths within the table; used pages inside the
-    pool; kv_len >= q_len when causal) in one synchronisation.  The messages
-    are those of ``prefill.py:194-233`` and ``paging.py:84-130``.  Returns the
-    longest query sequence."""
+def _check_paged_shapes(q, cache: PagedKVCache, cu_seqlens_q) -> None:
+    """The host-only checks of paged prefill; messages as in
+    ``prefill.py:194-233`` and ``paging.py:84-130``."""
     if not isinstance(cache, PagedKVCache):
         raise TypeError("cache must be a PagedKVCache")
     _check_layout(cache)
@@ -251,6 +299,12 @@ def _validate_paged(q, cache: PagedKVCache, cu_seqlens_q, causal) -> int:
     dev = q.device
     if any(t.device != dev for t in (cache.k_cache, cache.page_table, cache.seq_lens, cu_seqlens_q)):
         raise ValueError("q, the cache, its page table, seq_lens and cu_seqlens_q must live on one device")
+
+
+def _paged_stats(cache: PagedKVCache, cu_seqlens_q) -> list[int]:
+    """What ``_judge_paged`` checks, by torch reductions and one copy (CPU
+    tensors; ROCm tensors take the check kernel)."""
+    dev = cu_seqlens_q.device
     cq = cu_seqlens_q.to(torch.int64)
     lq = cq[1:] - cq[:-1]
     sl = cache.seq_lens.to(torch.int64)
@@ -267,7 +321,16 @@ def _validate_paged(q, cache: PagedKVCache, cu_seqlens_q, causal) -> int:
         cq[0], cq[-1], (lq < 0).any().to(torch.int64), lq.max(), (sl < lq).any().to(torch.int64),
         sl.min(), sl.max(), lo, hi, keyless.any().to(torch.int64), first_keyless, lq[first_keyless],
     ]).cpu().tolist()
-    q0, q_end, q_dec, max_q, short_kv, min_len, max_len, lo, hi, any_keyless, kl_b, kl_q = (int(x) for x in stats)
+    return [int(x) for x in stats]
+
+
+def _judge_paged(stats, q, cache: PagedKVCache, causal) -> int:
+    """The device-side checks (cu_seqlens_q monotone and ending at
+    q.shape[0]; lengths within the table; used pages inside the pool; kv_len
+    >= q_len when causal) on their numbers.  Returns the longest query
+    sequence."""
+    big = torch.iinfo(torch.int32).max
+    q0, q_end, q_dec, max_q, short_kv, min_len, max_len, lo, hi, any_keyless, kl_b, kl_q = stats
     if q0 != 0:
         raise ValueError("cu_seqlens must start at 0")
     if q_end != q.shape[0]:
@@ -301,6 +364,16 @@ def paged_prefill_launch(q: torch.Tensor, cache: PagedKVCache, cu_seqlens_q: tor
     the launch (long chunks copy their K/V rows there for the wide kernel);
     None or too small allocates one, so a caller that must not allocate
     (graph capture) passes its own."""
+    a, out, _keep = _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, out, kernel, rows,
+                                 workspace)
+    _hip.prefill_paged_with_args(a, _hip.current_stream_handle(q.device))
+    return out
+
+
+def _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, out=None, kernel=None, rows=None,
+                 workspace=None):
+    """The argument block of :func:`paged_prefill_launch`, its output, and
+    the tensors that have to live until the launch is enqueued."""
     if q.stride(-1) != 1 or cache.k_cache.stride(-1) != 1 or cache.v_cache.stride(-1) != 1:
         raise ValueError("q and the cache need a contiguous head_dim axis")
     if out is None:
@@ -318,8 +391,7 @@ def paged_prefill_launch(q: torch.Tensor, cache: PagedKVCache, cu_seqlens_q: tor
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace = workspace.data_ptr()
-    _hip.prefill_paged_with_args(a, _hip.current_stream_handle(q.device))
-    return out
+    return a, out, (q, pt, sl, cu, workspace)
 
 
 def paged_prefill_attention(
@@ -340,11 +412,42 @@ def paged_prefill_attention(
     :func:`prefill_attention` plus ``rows`` (store kind ``prefill_paged``).
     Returns ``q``'s shape and dtype.
     """
-    longest_q = _validate_paged(q, cache, cu_seqlens_q, causal)
+    _check_paged_shapes(q, cache, cu_seqlens_q)
+    check = block = error = None
+    if q.is_cuda and cache.page_table.numel() and _hip.is_loaded():
+        # as in prefill_attention: the check runs while the launch is prepared
+        stream = _hip.current_stream_handle(q.device)
+        cq = cu_seqlens_q if cu_seqlens_q.is_contiguous() else cu_seqlens_q.contiguous()
+        sl = cache.seq_lens if cache.seq_lens.is_contiguous() else cache.seq_lens.contiguous()
+        pt = cache.page_table if cache.page_table.stride(-1) == 1 else cache.page_table.contiguous()
+        check = _hip.check_begin(_hip.CHECK_PAGED, stream, q.device, cu_q=cq, seq_lens=sl, page_table=pt,
+                                 page_size=cache.page_size)
+        try:
+            block = _prepare_paged(q, cache, cq, max_seqlen_q, causal, softmax_scale, config)
+        except Exception as exc:
+            error = exc
+        r = check.wait()
+        flags, first = r[7], r[10]
+        stats = [r[3], r[4], flags & 1, r[8], flags & 4, r[0], r[1], r[12], r[13], first >= 0, first, r[11]]
+    else:
+        stats = _paged_stats(cache, cu_seqlens_q)
+    longest_q = _judge_paged(stats, q, cache, causal)
     if max_seqlen_q <= 0:
         raise ValueError(f"max_seqlen_q must be positive, got {max_seqlen_q}")
     if max_seqlen_q < longest_q:
         raise ValueError(f"max_seqlen_q {max_seqlen_q} is smaller than the longest query sequence {longest_q}")
+    if error is not None:
+        raise error
+    if block is None:
+        block = _prepare_paged(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, config)
+        stream = _hip.current_stream_handle(q.device)
+    a, out, _keep = block
+    _hip.prefill_paged_with_args(a, stream)
+    return out
+
+
+def _prepare_paged(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, config):
+    """:func:`_prepare` for :func:`paged_prefill_attention`."""
     if not q.is_cuda:
         raise RuntimeError("paged_prefill_attention: inputs must be ROCm device tensors; this build runs the "
                            "gfx950 HIP kernel only (no CPU or reference fallback)")
@@ -355,5 +458,5 @@ def paged_prefill_attention(
     cfg = _resolve_config(config, "prefill_paged", sig, defaults=PAGED_CONFIG)
     scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
     q = q if q.stride(-1) == 1 else q.contiguous()
-    return paged_prefill_launch(q, cache, cu_seqlens_q, int(max_seqlen_q), bool(causal), scale,
-                                kernel=cfg["kernel"], rows=cfg["rows"])
+    return _paged_block(q, cache, cu_seqlens_q, int(max_seqlen_q), bool(causal), scale, kernel=cfg["kernel"],
+                        rows=cfg["rows"])

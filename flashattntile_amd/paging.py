@@ -80,18 +80,26 @@ def _require(condition: bool, message: str) -> None:
 
 
 def _check_layout(cache: PagedKVCache) -> None:
-    """Host-only shape/dtype/device checks (no device synchronisation)."""
+    """Host-only shape/dtype/device checks (no device synchronisation).  The
+    messages are formatted only when a check fails: every decode call passes
+    here."""
     _require(isinstance(cache, PagedKVCache), "cache must be a PagedKVCache")
     k, v = cache.k_cache, cache.v_cache
-    _require(k.dim() == 4, f"k_cache must be 4-D [pages, page_size, kv_heads, dim], got {tuple(k.shape)}")
-    _require(k.shape == v.shape, f"k_cache {tuple(k.shape)} and v_cache {tuple(v.shape)} must match")
-    _require(k.dtype == v.dtype, f"k_cache dtype {k.dtype} != v_cache dtype {v.dtype}")
+    if k.dim() != 4:
+        raise AssertionError(f"k_cache must be 4-D [pages, page_size, kv_heads, dim], got {tuple(k.shape)}")
+    if k.shape != v.shape:
+        raise AssertionError(f"k_cache {tuple(k.shape)} and v_cache {tuple(v.shape)} must match")
+    if k.dtype != v.dtype:
+        raise AssertionError(f"k_cache dtype {k.dtype} != v_cache dtype {v.dtype}")
     _require(k.device == v.device, "k_cache and v_cache must live on the same device")
     _require(cache.page_size > 0, "page_size must be positive")
-    _require(k.shape[1] == cache.page_size, f"k_cache page dim {k.shape[1]} != page_size {cache.page_size}")
+    if k.shape[1] != cache.page_size:
+        raise AssertionError(f"k_cache page dim {k.shape[1]} != page_size {cache.page_size}")
     pt, sl = cache.page_table, cache.seq_lens
-    _require(pt.dtype == torch.int32, f"page_table must be int32, got {pt.dtype}")
-    _require(sl.dtype == torch.int32, f"seq_lens must be int32, got {sl.dtype}")
+    if pt.dtype != torch.int32:
+        raise AssertionError(f"page_table must be int32, got {pt.dtype}")
+    if sl.dtype != torch.int32:
+        raise AssertionError(f"seq_lens must be int32, got {sl.dtype}")
     _require(pt.dim() == 2, "page_table must be [batch, max_pages_per_seq]")
     _require(sl.dim() == 1, "seq_lens must be [batch]")
     _require(pt.shape[0] == sl.shape[0], "page_table and seq_lens batch dimensions disagree")
@@ -100,7 +108,7 @@ def _check_layout(cache: PagedKVCache) -> None:
 
 def cache_stats(cache: PagedKVCache, with_total_pages: bool = False) -> tuple[int, ...]:
     """``(min_len, max_len, min_page, max_page)`` in ONE device->host copy
-    (ROCm tensors: one ``fat_cache_stats`` launch; otherwise torch reductions).
+    (ROCm tensors: one check launch that the host polls; otherwise torch reductions).
 
     The page range covers ``page_table[:, :ceil(max_len / page_size)]`` for every
     row, the same entries ``paging.py:123-129`` inspects.  With no cached token
@@ -113,10 +121,10 @@ def cache_stats(cache: PagedKVCache, with_total_pages: bool = False) -> tuple[in
         return (0, 0, 0, -1, 0) if with_total_pages else (0, 0, 0, -1)
     big = torch.iinfo(torch.int32).max
     if sl.is_cuda and pt.is_cuda and sl.dtype == torch.int32 and pt.dtype == torch.int32 and \
-            sl.is_contiguous() and pt.dim() == 2 and pt.stride(-1) == 1:
+            sl.is_contiguous() and pt.dim() == 2 and pt.stride(-1) == 1 and pt.numel():
         from . import _hip
 
-        if _hip.is_loaded():  # one fused launch and one copy back (fat_cache_stats)
+        if _hip.is_loaded():  # one launch and one poll (fat_check_begin / fat_check_wait)
             stats = _hip.cache_stats(sl, pt, cache.page_size)
             if stats[2] == big:
                 stats[2], stats[3] = 0, -1
@@ -151,7 +159,12 @@ def validate_cache(cache: PagedKVCache, *, check_pages: bool = True) -> tuple[in
     ``(min_len, max_len)`` so callers need no further synchronisation.
     """
     _check_layout(cache)
-    min_len, max_len, lo, hi = cache_stats(cache)
+    return _judge_cache(cache, cache_stats(cache), check_pages)
+
+
+def _judge_cache(cache: PagedKVCache, stats: tuple[int, ...], check_pages: bool = True) -> tuple[int, int]:
+    """The device-side checks of :func:`validate_cache` on their numbers."""
+    min_len, max_len, lo, hi = stats
     _require(min_len >= 0, "seq_lens must be non-negative")
     capacity = cache.max_pages_per_seq * cache.page_size
     _require(max_len <= capacity, f"seq_len {max_len} exceeds page-table capacity {capacity}")
@@ -292,25 +305,29 @@ def _append_hip(cache: PagedKVCache, new_k: torch.Tensor, new_v: torch.Tensor, m
     if cache.batch_size == 0:
         return
     pt = cache.page_table if cache.page_table.stride(1) == 1 else cache.page_table.contiguous()
+    qk = qv = sk = sv = None
+    if mirror is not None:
+        qk, qv, sk, sv = mirror
+    stream = _hip.current_stream_handle(dev)
+    check = None
     if validate:
-        pos = cache.seq_lens.long()
-        block = torch.div(pos, cache.page_size, rounding_mode="floor")
-        rows = torch.arange(cache.batch_size, device=dev)
-        phys = pt[rows, block.clamp(0, cache.max_pages_per_seq - 1)]
-        min_len, max_pos, lo, hi = (int(x) for x in torch.stack(
-            [pos.min(), pos.max(), phys.min().long(), phys.max().long()]).cpu().tolist())
+        _require(cache.max_pages_per_seq > 0, f"append would exceed page-table capacity {cache.capacity}")
+        check = _hip.check_begin(_hip.CHECK_APPEND, stream, dev, seq_lens=cache.seq_lens, page_table=pt,
+                                 page_size=cache.page_size)
+    # prepared while the check kernel runs
+    nk = new_k if new_k.stride(2) == 1 else new_k.contiguous()
+    nv = new_v if new_v.stride(2) == 1 else new_v.contiguous()
+    args = _hip.append_args(nk, nv, cache.k_cache, cache.v_cache, pt, cache.seq_lens, cache.page_size, quant_k=qk,
+                            quant_v=qv, k_scale=sk, v_scale=sv, advance=True)
+    if check is not None:
+        r = check.wait()
+        min_len, max_pos, lo, hi = r[0], r[1], r[12], r[13]
         # Same checks, order and messages as validate_cache + paging.py:192-205.
         _require(min_len >= 0, "seq_lens must be non-negative")
         _require(max_pos <= cache.capacity, f"seq_len {max_pos} exceeds page-table capacity {cache.capacity}")
         _require(max_pos < cache.capacity, f"append would exceed page-table capacity {cache.capacity}")
         _require(lo >= 0 and hi < cache.num_pages, f"page_table maps to a page outside [0, {cache.num_pages})")
-    nk = new_k if new_k.stride(2) == 1 else new_k.contiguous()
-    nv = new_v if new_v.stride(2) == 1 else new_v.contiguous()
-    qk = qv = sk = sv = None
-    if mirror is not None:
-        qk, qv, sk, sv = mirror
-    _hip.append_kv(nk, nv, cache.k_cache, cache.v_cache, pt, cache.seq_lens, cache.page_size,
-                   quant_k=qk, quant_v=qv, k_scale=sk, v_scale=sv, advance=True)
+    _hip.append_with_args(args, stream)
 
 
 class AppendLaunch:

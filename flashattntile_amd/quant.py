@@ -26,7 +26,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .paging import PagedKVCache, validate_cache
+from .paging import PagedKVCache, _check_layout, _judge_cache, cache_stats
 
 __all__ = [
     "FP8_DTYPE",
@@ -101,6 +101,12 @@ def quantize_kv_pages(
 
     Returns ``(qk, qv, scale_k, scale_v, info)`` (``quant.py:84-142``).
     """
+    return _with_scale_range(*_quantize_kv_pages(k_cache, v_cache, mode))
+
+
+def _quantize_kv_pages(k_cache: torch.Tensor, v_cache: torch.Tensor, mode: str) -> tuple:
+    """:func:`quantize_kv_pages` without ``info``'s scale range (nothing
+    waits for the GPU)."""
     if k_cache.shape != v_cache.shape:
         raise ValueError(f"k/v shape mismatch: {tuple(k_cache.shape)} vs {tuple(v_cache.shape)}")
     if k_cache.dim() != 4:
@@ -141,10 +147,6 @@ def quantize_kv_pages(
 
     qk, k_scale = one(k_cache)
     qv, v_scale = one(v_cache)
-    if k_scale.numel():
-        scale_min, scale_max = (float(x) for x in torch.stack([k_scale.min(), k_scale.max()]).cpu().tolist())
-    else:
-        scale_min = scale_max = 0.0
     info = {
         "mode": mode,
         "dtype": str(qk.dtype),
@@ -154,10 +156,24 @@ def quantize_kv_pages(
         "num_kv_heads": int(kv_heads),
         "head_dim": int(head_dim),
         "scale_dtype": str(k_scale.dtype),
-        "scale_min": scale_min,
-        "scale_max": scale_max,
+        "scale_min": 0.0,
+        "scale_max": 0.0,
         "rounding": "round-to-nearest" if is_int8 else "cast-to-fp8",
     }
+    return qk, qv, k_scale, v_scale, info
+
+
+def _with_scale_range(qk: torch.Tensor, qv: torch.Tensor, k_scale: torch.Tensor, v_scale: torch.Tensor,
+                      info: dict) -> tuple:
+    """Fill ``info``'s range of the K scales (one host wait)."""
+    if k_scale.numel():
+        if k_scale.is_cuda:
+            from . import _hip
+
+            info["scale_min"], info["scale_max"] = _hip.float_range(k_scale)
+        else:
+            info["scale_min"], info["scale_max"] = (
+                float(x) for x in torch.stack([k_scale.min(), k_scale.max()]).tolist())
     return qk, qv, k_scale, v_scale, info
 
 
@@ -180,8 +196,30 @@ def dequantize_kv_pages(
 
 def quantize_cache(cache: PagedKVCache, mode: str = "auto") -> tuple[PagedKVCache, QuantScales]:
     """New cache holding quantised K/V (same table and lengths) plus scales."""
-    validate_cache(cache)
-    qk, qv, sk, sv, info = quantize_kv_pages(cache.k_cache, cache.v_cache, mode=mode)
+    _check_layout(cache)
+    # ROCm tensors: the quantisation, which reads neither the table nor the
+    # lengths, is enqueued behind their check instead of after its answer.
+    sl, pt = cache.seq_lens, cache.page_table
+    done = None
+    if cache.k_cache.is_cuda and sl.device == cache.k_cache.device and sl.is_contiguous() and pt.stride(1) == 1 \
+            and pt.numel():
+        from . import _hip
+
+        check = _hip.check_begin(_hip.CHECK_CACHE, _hip.current_stream_handle(sl.device), sl.device, seq_lens=sl,
+                                 page_table=pt, page_size=cache.page_size)
+        error = None
+        try:
+            done = _quantize_kv_pages(cache.k_cache, cache.v_cache, mode)
+        except Exception as exc:  # raised after the validation's own errors
+            error = exc
+        r = check.wait()
+        _judge_cache(cache, (r[0], r[1], r[12], r[13]))
+        if error is not None:
+            raise error
+    else:
+        _judge_cache(cache, cache_stats(cache))
+        done = _quantize_kv_pages(cache.k_cache, cache.v_cache, mode)
+    qk, qv, sk, sv, info = _with_scale_range(*done)
     quantized = PagedKVCache(k_cache=qk, v_cache=qv, page_table=cache.page_table,
                              seq_lens=cache.seq_lens, page_size=cache.page_size)
     return quantized, QuantScales(k=sk, v=sv, mode=info["mode"])

@@ -46,7 +46,9 @@
 extern "C" {
 #endif
 
-/* 14: fat_decode_args.merge_counters and fat_paged_decode_counters_bytes:
+/* 15: fat_check_begin / fat_check_wait (one launch and one host poll per
+ *     validated call).
+ * 14: fat_decode_args.merge_counters and fat_paged_decode_counters_bytes:
  *     split-K decode merges its partitions inside the decode launch.
  * 13: fat_cache_stats (paged-cache validation in one launch).
  * 12: fat_prefill_paged_args.workspace and
@@ -63,7 +65,7 @@ extern "C" {
  * 8: fp32 decode, any page size and head_dim 32/256 through the generic
  *    decode kernel (FAT_KERNEL_DECODE_GENERIC); the paged prefill `rows`
  *    field replaces the library's environment overrides. */
-#define FAT_ABI_VERSION 14
+#define FAT_ABI_VERSION 15
 
 /* Element types understood by the kernels. */
 enum fat_dtype {
@@ -491,6 +493,74 @@ typedef struct fat_cache_stats_args {
  * partition heuristic needs on `stream`; the caller copies `out` back and
  * checks it (one device-to-host copy per validation). */
 int fat_cache_stats(const fat_cache_stats_args* args, void* stream);
+
+/*
+ * The device-side numbers that a validated call checks before it launches
+ * (the lengths and page ids live on the GPU): one launch, whose workgroups
+ * write their results straight into host memory, and a host poll.  Between
+ * the two the caller prepares its launch.
+ *   kind FAT_CHECK_CACHE   seq_lens and the used page-table columns
+ *                          (flashattn_tile/paging.py:84-130)
+ *        FAT_CHECK_VARLEN  cu_q and cu_k (flashattn_tile/kernels/prefill.py:194-233)
+ *        FAT_CHECK_PAGED   cu_q, seq_lens and the used page-table columns
+ *        FAT_CHECK_APPEND  seq_lens and the page that each next token goes to
+ *                          (flashattn_tile/paging.py:191-205)
+ *        FAT_CHECK_RANGE   min and max of values[0 .. count - 1]
+ *                          (flashattn_tile/quant.py:128-142, the scale range)
+ *   host   int64 [FAT_CHECK_HOST_WORDS]: page-locked host memory that the
+ *          device can write, zero before its first use and used by one call
+ *          at a time
+ *   ticket positive, another value for each call with the same `host`
+ * Results (fat_check_wait's `result`, int64 [FAT_CHECK_RESULTS]):
+ *   0, 1   min and max of seq_lens
+ *   2      sum_b ceil(max(seq_lens[b], 0) / page_size)
+ *   3, 4   cu_q[0], cu_q[batch]
+ *   5, 6   cu_k[0], cu_k[batch]
+ *   7      1: cu_q decreases, 2: cu_k decreases, 4: some sequence holds fewer
+ *          keys than queries (key length: cu_k's, seq_lens[b] when PAGED)
+ *   8, 9   the longest query and (VARLEN) key length
+ *   10, 11 the first sequence with queries and no keys (-1: none), its queries
+ *   12, 13 min and max page id: over every row and the columns below
+ *          ceil(max(seq_lens) / page_size) (CACHE, PAGED; INT32_MAX and
+ *          INT32_MIN when no column is used), or of the entries
+ *          [b, clamp(floor(seq_lens[b] / page_size), 0, max_pages - 1)] (APPEND);
+ *          the bits of the fp32 min and max, NaN if a value is (RANGE)
+ * Entries that a kind doesn't name are undefined.
+ */
+enum fat_check_kind {
+  FAT_CHECK_CACHE = 0,
+  FAT_CHECK_VARLEN = 1,
+  FAT_CHECK_PAGED = 2,
+  FAT_CHECK_APPEND = 3,
+  FAT_CHECK_RANGE = 4
+};
+#define FAT_CHECK_RESULTS 16
+#define FAT_CHECK_MAX_GROUPS 64
+#define FAT_CHECK_HOST_WORDS (FAT_CHECK_RESULTS + 2 * FAT_CHECK_MAX_GROUPS)
+typedef struct fat_check_args {
+  const int32_t* cu_q;       /* [batch + 1] */
+  const int32_t* cu_k;       /* [batch + 1] */
+  const int32_t* seq_lens;   /* [batch] */
+  const int32_t* page_table; /* [batch, max_pages], row stride page_table_stride */
+  int64_t page_table_stride;
+  int64_t* host;
+  int64_t ticket;
+  int32_t kind;
+  int32_t batch;
+  int32_t max_pages;
+  int32_t page_size;
+  const float* values; /* [count], RANGE only */
+  int64_t count;
+} fat_check_args;
+
+/* Enqueue the check on `stream`.  FAT_E_LAUNCH while the stream is capturing
+ * (a validated call waits for the GPU, which a capture cannot). */
+int fat_check_begin(const fat_check_args* args, void* stream);
+
+/* Wait for the check that fat_check_begin enqueued with the same arguments
+ * and stream, and fill `result`.  Polls `host` for two milliseconds, then
+ * synchronises the stream. */
+int fat_check_wait(const fat_check_args* args, void* stream, int64_t* result);
 
 #ifdef __cplusplus
 }
