@@ -51,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "fat_last_error",
     "fat_paged_decode_workspace_bytes",
     "fat_paged_decode_counters_bytes",
+    "fat_paged_decode_balanced_workspace_bytes",
     "fat_paged_decode",
     "fat_paged_decode_noalloc",
     "fat_prefill_workspace_bytes",
@@ -114,6 +115,7 @@ class DecodeArgs(ctypes.Structure):
         ("q_len", _c_i32),
         ("kernel", _c_i32),
         ("merge_counters", _c_vp),
+        ("balanced", _c_i32),
     ]
 
 
@@ -335,6 +337,8 @@ def _load() -> None:
         lib.fat_last_error.restype = ctypes.c_char_p
         lib.fat_paged_decode_workspace_bytes.restype = ctypes.c_size_t
         lib.fat_paged_decode_workspace_bytes.argtypes = [_c_i32, _c_i32, _c_i32, _c_i32]
+        lib.fat_paged_decode_balanced_workspace_bytes.restype = ctypes.c_size_t
+        lib.fat_paged_decode_balanced_workspace_bytes.argtypes = [ctypes.POINTER(DecodeArgs)]
         lib.fat_paged_decode.restype = ctypes.c_int
         lib.fat_paged_decode.argtypes = [ctypes.POINTER(DecodeArgs), _c_vp]
         lib.fat_paged_decode_noalloc.restype = ctypes.c_int
@@ -532,6 +536,11 @@ def decode_workspace_bytes(batch: int, num_heads: int, head_dim: int, split_k: i
 def decode_counters_bytes(rows: int, num_heads: int) -> int:
     """Bytes of the split-K merge counters for ``rows`` = batch * q_len."""
     return int(lib().fat_paged_decode_counters_bytes(rows, num_heads))
+
+
+def decode_balanced_workspace_bytes(a: DecodeArgs) -> int:
+    """Workspace bytes of the launch of ``a`` when it runs balanced (0: it can't)."""
+    return int(lib().fat_paged_decode_balanced_workspace_bytes(ctypes.byref(a)))
 
 
 def prefill_workspace_bytes(total_k: int, num_kv_heads: int, head_dim: int) -> int:

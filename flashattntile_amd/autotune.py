@@ -44,6 +44,8 @@ __all__ = [
     "arithmetic_intensity",
     "decode_split_k",
     "decode_partition",
+    "decode_split",
+    "decode_balanced",
     "decode_heads_per_workgroup",
     "decode_signature",
     "prefill_signature",
@@ -207,6 +209,72 @@ def decode_partition(batch: int, num_heads: int, num_kv_heads: int, max_pages: i
             split = split + 1 if split < cap else split - 1
         chunk = math.ceil(max_pages / split)  # equal partitions of the longest sequence
     return int(max(1, split)), int(chunk)
+
+
+def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: int, mfma: bool = False,
+                 num_cus: int = MI355X_CUS) -> tuple[int, int | None]:
+    """``(split_k, waves)`` of a decode launch with ``split_k`` equal
+    partitions of every sequence: ``items`` (sequence, head group) pairs, each
+    one workgroup when it isn't split, over ``mean_len`` tokens on average and
+    ``max_len`` at most, ``item_token_bytes`` of K and V per token and head
+    group, on the MFMA kernel or a VALU one.  Waves None: the library's choice.
+
+    * As many partitions as fill the CUs once, no shorter than 128 tokens and
+      none below 256: a small launch is latency along its longest partition
+      (24 items of 2000 tokens 13.2 -> 10.0 us), a workgroup more than there
+      are CUs waits for a whole one, and the merge costs 1.5 us (35 items of
+      211 tokens 8.1 us whole, 8.9 in four).  To 16, which the decode launch
+      merges itself, unless those leave half the CUs idle over long sequences
+      (8 items of 40000 tokens 40.3 -> 33.9 us in 32).
+    * A CU streams at most 1.6 times its share of the memory rate (128
+      workgroups reach 5.2 of 6.2 TB/s).  Where a whole sequence takes one
+      more than 10 us, more partitions, until the longest of a ragged batch is
+      1.2 times a CU's share of the tokens and the CU with a workgroup more
+      than another has 1.4 times its share: 264 items of 1030-2793 tokens 71.2
+      -> 50.1 us, 128 of 1000-7900 with four queries each 66.9 -> 53.7.
+    * Eight waves where a CU has one workgroup, but four on the VALU kernels
+      for whole sequences below 1024 tokens (240 items of 609 tokens 17.3 ->
+      16.8 us, 33 x 8 of 68 11.4 -> 7.8) and in larger grids, except that the
+      library chooses for longer whole sequences.
+
+    Measured with 120 drawn batches against every split_k of 1-32 and both
+    numbers of waves; :func:`decode_partition`, which this replaces for the
+    library's own choice, was 1.1-2 times slower than the best of them.
+    """
+    items = max(1, int(items))
+    split = 1
+    if items < num_cus and max_len > 256:
+        cap = 16 if items <= 4 or max_len >= 4096 else 8
+        if 16 * items <= num_cus // 2 and max_len >= 4096:
+            cap = 64 if max_len >= 65536 else 32
+        split = max(1, min(num_cus // items, -(-max_len // 128), cap))
+    if max_len * item_token_bytes > 10 * 40e3:  # 40 GB/s per CU: bytes per us
+        if max_len >= 1.25 * mean_len and items * mean_len * item_token_bytes > 15 * 6.2e6:
+            need = max_len * num_cus / (1.2 * items * max(mean_len, 1.0))
+            if split < 0.7 * need:
+                split = min(math.ceil(need), 16, max(1, max_len // 256))
+        while split < min(8, max_len // 256) and items * split > num_cus // 2 \
+                and -(-items * split // num_cus) * num_cus > 1.4 * items * split:
+            split += 1
+        if num_cus // 2 < items * split < 4 * num_cus and (split > 1 or items < num_cus):
+            split = max(split, min(-(-4 * num_cus // items), 8, max_len // 512))
+    if items * split <= num_cus:
+        return split, 4 if not mfma and split == 1 and max_len < 1024 else 8
+    return split, None if not mfma and split == 1 and max_len >= 1024 else 4
+
+
+def decode_balanced(max_len: int, mean_len: float, kv_bytes: int, rows: int) -> bool:
+    """Whether a decode launch of the library's own choice cuts the batch into
+    equal runs (fat_decode_args.balanced) instead of :func:`decode_split`'s
+    partitions, where its kernel has that form: ragged batches whose K/V
+    (``kv_bytes``) take the memory 25 us or more, with at most 16 (head,
+    token) ``rows`` per workgroup.  64 sequences of 500-16000 tokens on an fp8
+    cache 151 -> 130.5 us, 64 log-uniform in [16, 65536] in fp16 403 -> 351,
+    40 of 100-10000 at head_dim 64 49.8 -> 46.5; level at 20 of 300-5000
+    (126 MB), and behind on uniform batches, which partitions divide as well
+    without finding their place in the batch first.
+    """
+    return max_len >= 1.5 * mean_len and kv_bytes >= 150e6 and rows <= 16
 
 
 def is_ragged(batch: int, max_pages: int, total_pages: int) -> bool:

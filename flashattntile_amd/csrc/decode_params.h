@@ -40,7 +40,16 @@ struct DecodeParams {
   // count (a power of two >= split_k, at most 16).
   int32_t* counters;
   int32_t smax;
+  // Balanced launches (decode_kernels.h): sequences of the batch, and rows of
+  // a workgroup's two partials in the workspace (ws_acc [W, 2, bal_rows, D],
+  // ws_ml [W, 2, bal_rows, 2]).
+  int32_t B, bal_rows;
 };
+
+// Limits of a balanced launch: sequences (their block counts are kept in LDS)
+// and (head, token) rows per workgroup (the last one merges alone).
+constexpr int kBalMaxSeqs = 1024;
+constexpr int kBalRows = 16;
 
 }  // namespace fat
 
@@ -54,5 +63,13 @@ constexpr int kGenericHeads = 8;
 // Returns FAT_OK or FAT_E_UNSUPPORTED / FAT_E_LAUNCH with the error set.
 int launch_decode_generic(const fat::DecodeParams& prm, int q_dtype, int kv, int head_dim, int heads_per_wg,
                           dim3 grid, hipStream_t stream);
+
+
+// Launch the balanced form (decode_balanced.hip) of the VALU kernel (lane: its
+// per-lane form), or for 8-bit caches without lane of the MFMA kernel, on
+// `groups` workgroups of four waves; the caller has checked that it is built
+// for the shape.
+int launch_decode_balanced(const fat::DecodeParams& prm, int q_dtype, int kv, bool lane, int head_dim, int groups,
+                           hipStream_t stream);
 
 }  // namespace fat_host

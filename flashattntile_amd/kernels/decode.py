@@ -35,7 +35,8 @@ import warnings
 import torch
 
 from .. import _hip
-from ..autotune import best_config, decode_partition, decode_signature, is_ragged
+from ..autotune import (best_config, decode_balanced, decode_partition, decode_signature, decode_split,
+                        is_ragged)
 from ..paging import PagedKVCache, _check_layout, cache_stats
 
 __all__ = [
@@ -60,7 +61,12 @@ __all__ = [
 # generic kernel is the library's own choice only for the shapes the VALU
 # kernel's per-lane form does not take either: head_dim 16 and 512, fp32 at
 # head_dim 256, 8-bit caches at head_dim 32, unaligned queries).
-DEFAULT_CONFIG = {"split_k": None, "num_warps": None, "num_stages": 2, "pages_per_split": None, "kernel": None}
+# balanced: 1 cuts the batch's work into equal runs, one per workgroup, in
+# place of split_k partitions per sequence, where the kernel has that form (n >
+# 1: with n workgroups; always of 4 waves), 0 doesn't; None: when split_k is None too, by
+# :func:`~flashattntile_amd.autotune.decode_balanced`.
+DEFAULT_CONFIG = {"split_k": None, "num_warps": None, "num_stages": 2, "pages_per_split": None, "kernel": None,
+                  "balanced": None}
 
 _KERNEL_CODES = {None: _hip.KERNEL_AUTO, "valu": _hip.KERNEL_DECODE_VALU, "mfma": _hip.KERNEL_DECODE_MFMA,
                  "generic": _hip.KERNEL_DECODE_GENERIC}
@@ -106,24 +112,67 @@ def resolve_decode_config(q: torch.Tensor, cache: PagedKVCache, max_len: int, to
     return _resolve_config(config, q, cache, max_len, total_pages, q_len)
 
 
+def _work_items(q: torch.Tensor, cache: PagedKVCache, kernel: str | None, q_len: int) -> tuple[int, int, bool, bool]:
+    """``(rows, items, mfma, balances)`` of a decode launch: the (query head,
+    token) rows of one workgroup, the (sequence, head group) pairs of the
+    batch, whether the library takes the MFMA kernel (``fat_paged_decode``),
+    and whether the kernel that it takes has a balanced form."""
+    group = int(q.shape[-2]) // cache.num_kv_heads
+    rows = group * q_len
+    quantized = cache.k_cache.dtype in _QUANT_DTYPES
+    d, page = cache.head_dim, cache.page_size
+    per_load = (4 if d == 128 else 8) * (2 if quantized else 1)  # rows that one 16-byte load per lane covers
+    fast = q.dtype != torch.float32 and d in (64, 128) and page >= per_load and page & (page - 1) == 0
+    if fast:
+        per_wg = 32 if kernel == "mfma" or (kernel is None and (quantized or group >= 8)) or q_len > 1 else \
+            (8 if group >= 8 else 4)
+        balances = quantized if per_wg == 32 else per_wg == 4
+    else:  # the per-lane form, else the generic kernel
+        per_wg = 4
+        balances = d >= (64 if quantized else 32) and d <= (256 if quantized else 128)
+    if kernel == "generic":
+        per_wg, balances = 8, False
+    return min(rows, per_wg), int(q.shape[0]) * cache.num_kv_heads * -(-rows // per_wg), per_wg == 32, balances
+
+
 def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: int, total_pages: int,
                   q_len: int) -> dict:
     resolved = dict(DEFAULT_CONFIG)
     resolved.update(config)
+    waves = resolved["num_warps"]
     if resolved["split_k"] is None:
-        max_pages = -(-max_len // cache.page_size)
-        split, chunk = decode_partition(int(q.shape[0]), int(q.shape[-2]), cache.num_kv_heads, max_pages,
-                                        total_pages, quantized=cache.k_cache.dtype in _QUANT_DTYPES, q_len=q_len)
-        resolved["split_k"] = split
-        if resolved["pages_per_split"] is None:
-            resolved["pages_per_split"] = chunk
-        # A skewed batch runs 4-wave workgroups: the library's own choice (8
-        # waves for partitions of >= 1024 keys, measured on uniform batches)
-        # was 1.04-1.4x slower on the skewed batches of decode_partition.
-        if resolved["num_warps"] is None and is_ragged(int(q.shape[0]), max_pages, total_pages):
-            resolved["num_warps"] = 4
+        batch, heads, hkv, page = int(q.shape[0]), int(q.shape[-2]), cache.num_kv_heads, cache.page_size
+        max_pages = -(-max_len // page)
+        k = cache.k_cache
+        rows, items, mfma, balances = _work_items(q, cache, resolved["kernel"], q_len)
+        mean_len = min(max_len, total_pages * page / max(1, batch))
+        token_bytes = 2 * cache.head_dim * k.element_size()
+        if resolved["balanced"] is None and resolved["pages_per_split"] is None and waves in (None, 4) \
+                and balances:
+            resolved["balanced"] = int(decode_balanced(max_len, mean_len, token_bytes * hkv * total_pages * page,
+                                                       rows))
+        if resolved["balanced"] or resolved["pages_per_split"] is not None:
+            # what a kernel without the balanced form falls back to
+            split, chunk = decode_partition(batch, heads, hkv, max_pages, total_pages,
+                                            quantized=k.dtype in _QUANT_DTYPES, q_len=q_len)
+            resolved["split_k"] = split
+            if resolved["pages_per_split"] is None:
+                resolved["pages_per_split"] = chunk
+            # A skewed batch cut into partitions of one size runs 4-wave
+            # workgroups: the library's own choice (8 waves for partitions of
+            # >= 1024 keys, measured on uniform batches) was 1.04-1.4x slower.
+            if resolved["num_warps"] is None and is_ragged(batch, max_pages, total_pages):
+                resolved["num_warps"] = 4
+        else:
+            resolved["split_k"], chosen = decode_split(items, max_len, mean_len, token_bytes, mfma)
+            resolved["pages_per_split"] = 0
+            if resolved["num_warps"] is None:
+                resolved["num_warps"] = chosen
     if resolved["pages_per_split"] is None:
         resolved["pages_per_split"] = 0
+    balanced = resolved["balanced"] = resolved["balanced"] or 0
+    if not isinstance(balanced, int) or not 0 <= balanced <= 4096:
+        raise ValueError(f"balanced must be an integer in [0, 4096], got {balanced}")
     split_k = resolved["split_k"]
     if not isinstance(split_k, int) or isinstance(split_k, bool) or split_k < 1:
         raise ValueError(f"split_k must be a positive integer, got {split_k}")
@@ -313,6 +362,20 @@ def _launch_block(a, q, split_k, workspace=None, waves_per_group=None, pages_per
     _hip.decode_with_args(a, _hip.current_stream_handle(q.device))
 
 
+def _balance(a, cfg) -> int:
+    """Set up the block ``a`` for a balanced launch if ``cfg`` asks for one and
+    the kernel has that form; returns its workspace bytes (0: it hasn't, and
+    the block is for split_k partitions)."""
+    if not cfg["balanced"]:
+        return 0
+    a.kernel = _KERNEL_CODES[cfg["kernel"]]
+    a.balanced = cfg["balanced"]
+    need = _hip.decode_balanced_workspace_bytes(a)
+    if not need:
+        a.balanced = 0
+    return need
+
+
 def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     """Launch with the resolved partitions, from the prepared block if there
     is one."""
@@ -320,6 +383,14 @@ def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     if prepared is None:
         prepared = _decode_block(q, cache, scale, scales)
     a, out, keep = prepared
+    need = _balance(a, cfg)
+    if need:
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        a.workspace = workspace.data_ptr()
+        a.merge_counters = merge_counters(q, 2).data_ptr()
+        _hip.decode_with_args(a, _hip.current_stream_handle(q.device))
+        del keep
+        return out
     _launch_block(a, q, cfg["split_k"], waves_per_group=cfg["num_warps"], pages_per_split=cfg["pages_per_split"],
                   kernel=cfg["kernel"], counters=merge_counters(q, cfg["split_k"]))
     del keep
@@ -505,22 +576,25 @@ class DecodeLaunch:
         self.config = cfg
         self.softmax_scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
         rows = q.shape[0] * q_len
-        need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], cfg["split_k"])
+        self._args = _hip.decode_args(q, cache.k_cache, cache.v_cache, cache.page_table, cache.seq_lens, q,
+                                      cache.page_size, self.softmax_scale, cfg["split_k"], k_scale=k_scale,
+                                      v_scale=v_scale, waves_per_group=cfg["num_warps"] or 0,
+                                      pages_per_split=cfg["pages_per_split"], kernel=_KERNEL_CODES[cfg["kernel"]])
+        need = _balance(self._args, cfg)
+        merged = bool(need) or cfg["split_k"] > 1
+        if not need:
+            need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], cfg["split_k"])
         self.workspace = torch.empty(max(1, need), dtype=torch.uint8, device=q.device) if need else None
-        # Zeroed split-K merge counters of this launch (each run leaves them
-        # zero): the decode kernel merges its partitions itself.  Runs of one
+        # Zeroed merge counters of this launch (each run leaves them zero):
+        # the decode kernel merges its partitions itself.  Runs of one
         # DecodeLaunch share them, as they share the workspace.
         self.counters = (torch.zeros(_hip.decode_counters_bytes(rows, q.shape[-2]) // 4, dtype=torch.int32,
-                                     device=q.device) if cfg["split_k"] > 1 else None)
+                                     device=q.device) if merged else None)
+        self._args.workspace = None if self.workspace is None else self.workspace.data_ptr()
+        self._args.merge_counters = None if self.counters is None else self.counters.data_ptr()
         self._keep = (cache, k_scale, v_scale)  # the argument block points into these
         self._shape, self._dtype = tuple(q.shape), q.dtype
         self._device = q.device
-        self._args = _hip.decode_args(q, cache.k_cache, cache.v_cache, cache.page_table, cache.seq_lens, q,
-                                      cache.page_size, self.softmax_scale, cfg["split_k"],
-                                      workspace=self.workspace, k_scale=k_scale, v_scale=v_scale,
-                                      waves_per_group=cfg["num_warps"] or 0,
-                                      pages_per_split=cfg["pages_per_split"], kernel=_KERNEL_CODES[cfg["kernel"]],
-                                      counters=self.counters)
 
     def run(self, q: torch.Tensor, out: torch.Tensor | None = None, stream: int | None = None) -> torch.Tensor:
         """Decode ``q`` into ``out`` (default: a new tensor) on ``stream``

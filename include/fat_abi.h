@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-/* 15: fat_check_begin / fat_check_wait (one launch and one host poll per
+/* 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
  *     validated call).
  * 14: fat_decode_args.merge_counters and fat_paged_decode_counters_bytes:
  *     split-K decode merges its partitions inside the decode launch.
@@ -211,6 +211,14 @@ typedef struct fat_decode_args {
    * merges and the counters are not touched.  Launches that may run at the
    * same time (other streams) must not share counters. */
   int32_t* merge_counters;
+  /* > 0: cut the batch's work into equal runs, one per workgroup, instead of
+   * split_k partitions per sequence, where the kernel that takes the launch
+   * has that form (fat_paged_decode_balanced_workspace_bytes is non-zero),
+   * merge_counters are given and `workspace` holds that many bytes; split_k
+   * and waves_per_group are then not read.  1: the library's number of
+   * workgroups, else that many (to 4096).  Where it hasn't, split_k
+   * partitions as with 0. */
+  int32_t balanced;
 } fat_decode_args;
 
 /*
@@ -403,6 +411,11 @@ const char* fat_last_error(void);
 /* Bytes of split-K workspace fat_paged_decode needs (0 when split_k == 1). */
 size_t fat_paged_decode_workspace_bytes(int32_t batch, int32_t num_heads,
                                         int32_t head_dim, int32_t split_k);
+
+/* Bytes of workspace that the launch described by `args` uses when it runs
+ * balanced (fat_decode_args.balanced), 0 when it can't.  Reads the sizes,
+ * types, strides and query address; no device access. */
+size_t fat_paged_decode_balanced_workspace_bytes(const fat_decode_args* args);
 
 /* Bytes of fat_decode_args.merge_counters for `rows` = batch * q_len query
  * rows (q_len 1 for single-query decode) of num_heads heads. */
