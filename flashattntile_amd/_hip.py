@@ -21,7 +21,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libfat_hip.so"
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 # enum fat_dtype
 DT_F16 = 0
@@ -58,6 +58,7 @@ EXPORTED_SYMBOLS = (
     "fat_prefill_varlen_workspace_bytes",
     "fat_prefill_varlen",
     "fat_prefill_paged_workspace_bytes",
+    "fat_prefill_paged_v_bytes",
     "fat_prefill_paged",
     "fat_quantize_pages",
     "fat_append_kv",
@@ -190,6 +191,7 @@ class PrefillPagedArgs(ctypes.Structure):
         ("kernel", _c_i32),
         ("rows", _c_i32),
         ("workspace", _c_vp),
+        ("v_workspace", _c_vp),
     ]
 
 
@@ -351,6 +353,8 @@ def _load() -> None:
         lib.fat_prefill_varlen.argtypes = [ctypes.POINTER(PrefillArgs), _c_vp]
         lib.fat_prefill_paged_workspace_bytes.restype = ctypes.c_size_t
         lib.fat_prefill_paged_workspace_bytes.argtypes = [ctypes.POINTER(PrefillPagedArgs)]
+        lib.fat_prefill_paged_v_bytes.restype = ctypes.c_size_t
+        lib.fat_prefill_paged_v_bytes.argtypes = [ctypes.POINTER(PrefillPagedArgs)]
         lib.fat_prefill_paged.restype = ctypes.c_int
         lib.fat_prefill_paged.argtypes = [ctypes.POINTER(PrefillPagedArgs), _c_vp]
         lib.fat_quantize_pages.restype = ctypes.c_int
@@ -736,6 +740,11 @@ def prefill_args(
 def prefill_paged_workspace_bytes(a: PrefillPagedArgs) -> int:
     """Workspace bytes the paged launch of ``a`` uses (0: it runs without one)."""
     return int(lib().fat_prefill_paged_workspace_bytes(ctypes.byref(a)))
+
+
+def prefill_paged_v_bytes(a: PrefillPagedArgs) -> int:
+    """Bytes of the fp16 copy of V that the paged launch of ``a`` uses (0: none)."""
+    return int(lib().fat_prefill_paged_v_bytes(ctypes.byref(a)))
 
 
 def prefill_paged_with_args(a: PrefillPagedArgs, stream: int) -> None:

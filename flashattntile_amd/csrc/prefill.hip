@@ -1079,53 +1079,90 @@ void prefill_pp_kernel(const PrefillParams p) {
 // fp16 inf and NaN.
 //
 // The pre-pass walks each sequence in 64-row tiles that start at the
-// sequence's first row.  Tile t of sequence b records its maximum in slot
+// sequence's first row.  It converts them with s = 0 and records each tile's
+// largest exponent, so V is read once; a second launch takes every (sequence,
+// KV head)'s maximum and converts again the few that need another scale (read
+// first and converted after, as two launches: 12.4 us where this takes
+// 11.3; 8192 keys, 8 heads).  Tile t of a packed sequence b has slot
 // b + floor(cu_k[b] / 64) + t of its head's row of `tilemax`: consecutive
 // sequences never share a slot, and every slot is below nblk + B (nblk =
-// ceil(total_k / 64)).
+// ceil(total_k / 64)).  Paged, sequence b's copy starts at row b cap and its
+// slots at b ceil(cap / 64), with cap = max_pages * page_size.
 // ---------------------------------------------------------------------------
 constexpr int kVpreRows = 64;  // V rows per pre-pass tile
 
-// Rows [r0, r1) of sequence b (clamped into [0, total_k)) and its tile count.
+// Rows [r0, r1) of sequence b in the copy (packed: clamped into [0, total_k))
+// and its tiles.
 struct VpreSeq {
-  int r0, r1, ntiles, slot0;
+  int64_t r0, r1;
+  int ntiles, slot0;
 };
-__device__ __forceinline__ VpreSeq vpre_seq(const int32_t* __restrict__ cu_k, int b, int total_k, int nslot) {
+template <bool PAGED>
+__device__ __forceinline__ VpreSeq vpre_seq(const PrefillParams& p, int b, int total_k, int nslot) {
   VpreSeq s;
-  s.r0 = min(max(cu_k[b], 0), total_k);
-  s.r1 = min(max(cu_k[b + 1], s.r0), total_k);
-  s.ntiles = (s.r1 - s.r0 + kVpreRows - 1) / kVpreRows;
-  s.slot0 = b + s.r0 / kVpreRows;
+  if constexpr (PAGED) {
+    const int cap = p.max_pages << p.pshift;
+    s.r0 = (int64_t)b * cap;
+    s.r1 = s.r0 + min(max(p.lens[b], 0), cap);
+    s.slot0 = b * ((cap + kVpreRows - 1) / kVpreRows);
+  } else {
+    s.r0 = min(max(p.cu_k[b], 0), total_k);
+    s.r1 = min(max(p.cu_k[b + 1], (int)s.r0), total_k);
+    s.slot0 = b + (int)s.r0 / kVpreRows;
+  }
+  s.ntiles = (int)(s.r1 - s.r0 + kVpreRows - 1) / kVpreRows;
   s.ntiles = min(s.ntiles, max(nslot - s.slot0, 0));  // in range for any cu_k
   return s;
 }
+// Chunk ch of head h of row `row` (in the copy's order) of sequence b.
+template <bool PAGED>
+__device__ __forceinline__ u32x4 vpre_load(const PrefillParams& p, const VpreSeq& sq, int b, int h, int64_t row, int ch) {
+  int64_t o = (int64_t)h * p.v_sh + 8 * ch;
+  if constexpr (PAGED) {
+    const int key = (int)(row - sq.r0);
+    const int page = min(max(p.pt[(int64_t)b * p.pt_sb + (key >> p.pshift)], 0), p.num_pages - 1);
+    o += (int64_t)page * p.v_sp + (int64_t)(key & ((1 << p.pshift) - 1)) * p.v_st;
+  } else {
+    o += row * p.v_st;
+  }
+  return *reinterpret_cast<const u32x4*>(p.v + 2 * o);
+}
 
-// Largest finite bf16 exponent field of |v| over tile t of sequence b, KV
-// head h -> tilemax[h * nslot + slot].  Grid (x, Hkv, B); workgroup x takes
-// tiles x, x + gridDim.x, ...
-template <int D>
-__global__ __launch_bounds__(256) void bf16v_expmax_kernel(const uint16_t* __restrict__ v, int64_t v_st,
-                                                           int64_t v_sh, const int32_t* __restrict__ cu_k,
-                                                           int total_k, int nslot,
-                                                           int32_t* __restrict__ tilemax) {
+// fp16(v) of the tiles of sequence b, KV head h, into the dense [rows, Hkv, D]
+// array v16, and the largest finite bf16 exponent field of |v| over each tile
+// -> tilemax[h * nslot + slot].  Grid (x, Hkv, B); workgroup x takes tiles x, x
+// + gridDim.x, ...
+template <int D, bool PAGED>
+__global__ __launch_bounds__(256) void bf16v_to_f16_kernel(const PrefillParams p, int total_k, int nslot,
+                                                           int32_t* __restrict__ tilemax,
+                                                           uint16_t* __restrict__ v16) {
   constexpr int CPR = D / 8;  // 16-byte chunks per row
+  constexpr int N = kVpreRows * CPR / 256;
   const int h = blockIdx.y;
   const int b = blockIdx.z;
-  const VpreSeq sq = vpre_seq(cu_k, b, total_k, nslot);
+  const VpreSeq sq = vpre_seq<PAGED>(p, b, total_k, nslot);
   __shared__ u32 red[4];
   for (int t = blockIdx.x; t < sq.ntiles; t += gridDim.x) {
     u32 em = 0;
-    for (int c = threadIdx.x; c < kVpreRows * CPR; c += 256) {
-      const int row = sq.r0 + t * kVpreRows + c / CPR;
-      if (row < sq.r1) {
-        const u32x4 x =
-            *reinterpret_cast<const u32x4*>(v + (int64_t)row * v_st + (int64_t)h * v_sh + 8 * (c % CPR));
+    u32x4 x[N];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const u32 lo = x[e] & 0x7f80u, hi = (x[e] >> 16) & 0x7f80u;
-          em = max(em, max(lo == 0x7f80u ? 0u : lo, hi == 0x7f80u ? 0u : hi));
-        }
+    for (int i = 0; i < N; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      const int64_t row = sq.r0 + (int64_t)t * kVpreRows + c / CPR;
+      x[i] = row < sq.r1 ? vpre_load<PAGED>(p, sq, b, h, row, c % CPR) : u32x4{0u, 0u, 0u, 0u};
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      const int64_t row = sq.r0 + (int64_t)t * kVpreRows + c / CPR;
+      u32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32 lo = x[i][e] & 0x7f80u, hi = (x[i][e] >> 16) & 0x7f80u;
+        em = max(em, max(lo == 0x7f80u ? 0u : lo, hi == 0x7f80u ? 0u : hi));
+        y[e] = Pair<F16>::pack(Pair<BF16>::lo(x[i][e]), Pair<BF16>::hi(x[i][e]));
       }
+      if (row < sq.r1) *reinterpret_cast<u32x4*>(v16 + (row * p.Hkv + h) * D + 8 * (c % CPR)) = y;
     }
     u32 m = em;
 #pragma unroll
@@ -1138,20 +1175,18 @@ __global__ __launch_bounds__(256) void bf16v_expmax_kernel(const uint16_t* __res
   }
 }
 
-// fp16(v * 2^-s) of the tiles of sequence b, KV head h, into the dense
-// [total_k, Hkv, D] array v16, where s is the (b, h) scale taken from that
-// sequence's tile maxima; workgroup (0, h, b) records s in
+// The scale s of sequence b, KV head h from its tile maxima; where it isn't 0,
+// fp16(v * 2^-s) of its tiles into v16.  Workgroup (0, h, b) records s in
 // seq_scale[b * Hkv + h] (0 for a sequence without keys).
-template <int D>
-__global__ __launch_bounds__(256) void bf16v_to_f16_kernel(const uint16_t* __restrict__ v, int64_t v_st, int64_t v_sh,
-                                                           const int32_t* __restrict__ cu_k, int total_k, int Hkv,
-                                                           int nslot, const int32_t* __restrict__ tilemax,
-                                                           uint16_t* __restrict__ v16,
-                                                           int32_t* __restrict__ seq_scale) {
+template <int D, bool PAGED>
+__global__ __launch_bounds__(256) void bf16v_rescale_kernel(const PrefillParams p, int total_k, int nslot,
+                                                            const int32_t* __restrict__ tilemax,
+                                                            uint16_t* __restrict__ v16,
+                                                            int32_t* __restrict__ seq_scale) {
   constexpr int CPR = D / 8;
   const int h = blockIdx.y;
   const int b = blockIdx.z;
-  const VpreSeq sq = vpre_seq(cu_k, b, total_k, nslot);
+  const VpreSeq sq = vpre_seq<PAGED>(p, b, total_k, nslot);
   int le = 0;
   for (int i = threadIdx.x; i < sq.ntiles; i += 256) le = max(le, tilemax[(int64_t)h * nslot + sq.slot0 + i]);
   __shared__ int red[4];
@@ -1161,17 +1196,18 @@ __global__ __launch_bounds__(256) void bf16v_to_f16_kernel(const uint16_t* __res
   __syncthreads();
   le = max(max(red[0], red[1]), max(red[2], red[3]));
   const int sw = max(0, le - 141);  // 2^(le - 127) >= 2^15 <=> le >= 142; finite le <= 254
-  if (blockIdx.x == 0 && threadIdx.x == 0) seq_scale[b * Hkv + h] = sw;
+  if (blockIdx.x == 0 && threadIdx.x == 0) seq_scale[b * p.Hkv + h] = sw;
+  if (sw == 0) return;
   const float f = as_f32((u32)(127 - sw) << 23);  // 2^-sw, sw <= 113
   for (int t = blockIdx.x; t < sq.ntiles; t += gridDim.x) {
     for (int c = threadIdx.x; c < kVpreRows * CPR; c += 256) {
-      const int row = sq.r0 + t * kVpreRows + c / CPR;
+      const int64_t row = sq.r0 + (int64_t)t * kVpreRows + c / CPR;
       if (row >= sq.r1) continue;
-      const u32x4 x = *reinterpret_cast<const u32x4*>(v + (int64_t)row * v_st + (int64_t)h * v_sh + 8 * (c % CPR));
+      const u32x4 x = vpre_load<PAGED>(p, sq, b, h, row, c % CPR);
       u32x4 y;
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = Pair<F16>::pack(Pair<BF16>::lo(x[e]) * f, Pair<BF16>::hi(x[e]) * f);
-      *reinterpret_cast<u32x4*>(v16 + ((int64_t)row * Hkv + h) * D + 8 * (c % CPR)) = y;
+      *reinterpret_cast<u32x4*>(v16 + (row * p.Hkv + h) * D + 8 * (c % CPR)) = y;
     }
   }
 }
@@ -1336,6 +1372,56 @@ size_t vpre_need(PrefillKind kind, int dtype, int64_t B, int64_t Hkv, int D, int
   return vpre_bytes_v16(total_k, Hkv, D) + (size_t)(Hkv * (nblk + 2 * B)) * sizeof(int32_t);
 }
 
+// The MFMA kernels take a positive scale: a negative one runs as its
+// magnitude with Q's signs flipped as Q is loaded (exact in fp16/bf16 and
+// through the MFMA sums), a zero one with Q zeroed (every logit 0).
+void fold_scale(fat::PrefillParams& prm, float softmax_scale) {
+  prm.q_and = ~0u;
+  prm.q_xor = 0u;
+  prm.scale_log2 = softmax_scale * fat::kLog2e;
+  if (softmax_scale < 0.f) {
+    prm.q_xor = 0x80008000u;
+    prm.scale_log2 = -prm.scale_log2;
+  } else if (softmax_scale == 0.f) {
+    prm.q_and = 0u;
+    prm.scale_log2 = fat::kLog2e;
+  }
+}
+
+// Packs of 2-16 sequences run their (query block, sequence) items on the wide
+// kernel longest chain first (the kernel ranks them: O(B) per thread, at most
+// 512 items, one per thread).
+void rank_wide_items(fat::PrefillParams& prm) {
+  const int64_t items = (int64_t)prm.nqb * prm.B;
+  prm.rank_items = (prm.B >= 2 && prm.B <= fat::kWideRankMaxSeqs && items <= fat::kWideBM) ? (int)items : 0;
+}
+
+// Converts bf16 V to fp16 into `workspace` (the layout of vpre_need) and points
+// prm's V at the copy.  One workgroup per tile of the longest sequence
+// (max_seqlen_k bounds the tile count; a workgroup loops over the tiles beyond
+// gridDim.x anyway); the second launch has nothing but maxima to read as a
+// rule, so it has no more than the CUs hold (2048), or 8 per (sequence, head).
+template <int D, bool PAGED>
+int launch_vpre(fat::PrefillParams& prm, int64_t rows, int nslot, int64_t max_seqlen_k, void* workspace,
+                hipStream_t stream) {
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  uint16_t* v16 = reinterpret_cast<uint16_t*>(ws);
+  int32_t* tilemax = reinterpret_cast<int32_t*>(ws + vpre_bytes_v16(rows, prm.Hkv, D));
+  int32_t* seq_scale = tilemax + (int64_t)prm.Hkv * nslot;
+  const int64_t tiles = (max_seqlen_k + fat::kVpreRows - 1) / fat::kVpreRows;
+  const unsigned x = (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 65535));
+  const unsigned x2 = (unsigned)std::max<int64_t>(8, 2048 / ((int64_t)prm.Hkv * prm.B));
+  hipLaunchKernelGGL((fat::bf16v_to_f16_kernel<D, PAGED>), dim3(x, (unsigned)prm.Hkv, (unsigned)prm.B), dim3(256), 0,
+                     stream, prm, (int)rows, nslot, tilemax, v16);
+  hipLaunchKernelGGL((fat::bf16v_rescale_kernel<D, PAGED>), dim3(std::min(x, x2), (unsigned)prm.Hkv, (unsigned)prm.B),
+                     dim3(256), 0, stream, prm, (int)rows, nslot, tilemax, v16, seq_scale);
+  prm.v = reinterpret_cast<const uint8_t*>(v16);
+  prm.v_st = (int64_t)prm.Hkv * D;
+  prm.v_sh = D;
+  prm.v_head_scale = seq_scale;
+  return fat_host::launch_status("bf16v_to_f16_kernel");
+}
+
 template <int PG>
 int launch_prefill(fat::PrefillParams& prm, int max_seqlen_q, int64_t max_seqlen_k, int dtype, int D, bool causal,
                    float softmax_scale, int kernel, const char* who, hipStream_t stream, void* workspace = nullptr,
@@ -1379,19 +1465,7 @@ int launch_prefill(fat::PrefillParams& prm, int max_seqlen_q, int64_t max_seqlen
   }
   const int bm = kind == PF_WIDE ? fat::kWideBM : kind == PF_PINGPONG ? fat::kPBM : fat::kBM;
   prm.nqb = (max_seqlen_q + bm - 1) / bm;
-  // The MFMA kernels take a positive scale: a negative one runs as its
-  // magnitude with Q's signs flipped as Q is loaded (exact in fp16/bf16 and
-  // through the MFMA sums), a zero one with Q zeroed (every logit 0).
-  prm.q_and = ~0u;
-  prm.q_xor = 0u;
-  prm.scale_log2 = softmax_scale * fat::kLog2e;
-  if (softmax_scale < 0.f) {
-    prm.q_xor = 0x80008000u;
-    prm.scale_log2 = -prm.scale_log2;
-  } else if (softmax_scale == 0.f) {
-    prm.q_and = 0u;
-    prm.scale_log2 = fat::kLog2e;
-  }
+  fold_scale(prm, softmax_scale);
   const int64_t n = (int64_t)prm.nqb * prm.B * prm.H;
   if (n > 0x7fffffff) {
     fat_host::set_error("%s: too many query blocks (%lld)", who, (long long)n);
@@ -1402,49 +1476,15 @@ int launch_prefill(fat::PrefillParams& prm, int max_seqlen_q, int64_t max_seqlen
   // when the caller gave the workspace.
   prm.v_head_scale = nullptr;
   if (PG == 0 && workspace && vpre_need(kind, dtype, prm.B, prm.Hkv, D, total_q, total_k, max_seqlen_k) > 0) {
-    const int nblk = (total_k + fat::kVpreRows - 1) / fat::kVpreRows;
-    const int nslot = nblk + prm.B;
-    uint8_t* ws = static_cast<uint8_t*>(workspace);
-    uint16_t* v16 = reinterpret_cast<uint16_t*>(ws);
-    int32_t* tilemax = reinterpret_cast<int32_t*>(ws + vpre_bytes_v16(total_k, prm.Hkv, D));
-    int32_t* seq_scale = tilemax + (int64_t)prm.Hkv * nslot;
-    // One workgroup per tile of the longest sequence (max_seqlen_k bounds the
-    // tile count; a workgroup loops over the tiles beyond gridDim.x anyway).
-    const int64_t tiles = (max_seqlen_k + fat::kVpreRows - 1) / fat::kVpreRows;
-    const dim3 pgrid((unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 65535)), (unsigned)prm.Hkv,
-                     (unsigned)prm.B);
-    const uint16_t* vsrc = reinterpret_cast<const uint16_t*>(prm.v);
-    const int32_t* cuk = prm.cu_k;
-    if (D == 128) {
-      hipLaunchKernelGGL((fat::bf16v_expmax_kernel<128>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, nslot, tilemax);
-      hipLaunchKernelGGL((fat::bf16v_to_f16_kernel<128>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, prm.Hkv, nslot, tilemax, v16, seq_scale);
-    } else if (D == 64) {
-      hipLaunchKernelGGL((fat::bf16v_expmax_kernel<64>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, nslot, tilemax);
-      hipLaunchKernelGGL((fat::bf16v_to_f16_kernel<64>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, prm.Hkv, nslot, tilemax, v16, seq_scale);
-    } else {
-      hipLaunchKernelGGL((fat::bf16v_expmax_kernel<32>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, nslot, tilemax);
-      hipLaunchKernelGGL((fat::bf16v_to_f16_kernel<32>), pgrid, dim3(256), 0, stream, vsrc, prm.v_st, prm.v_sh,
-                         cuk, total_k, prm.Hkv, nslot, tilemax, v16, seq_scale);
-    }
-    const int rc = fat_host::launch_status("bf16v_to_f16_kernel");
+    const int nslot = (total_k + fat::kVpreRows - 1) / fat::kVpreRows + prm.B;
+    const int rc = D == 128  ? launch_vpre<128, false>(prm, total_k, nslot, max_seqlen_k, workspace, stream)
+                   : D == 64 ? launch_vpre<64, false>(prm, total_k, nslot, max_seqlen_k, workspace, stream)
+                             : launch_vpre<32, false>(prm, total_k, nslot, max_seqlen_k, workspace, stream);
     if (rc != FAT_OK) return rc;
-    prm.v = reinterpret_cast<const uint8_t*>(v16);
-    prm.v_st = (int64_t)prm.Hkv * D;
-    prm.v_sh = D;
-    prm.v_head_scale = seq_scale;
   }
   if (kind == PF_WIDE) {
-    // Packs of 2-16 sequences run their (query block, sequence) items
-    // longest chain first (the kernel ranks them: O(B) per thread, at most
-    // 512 items, one per thread).
-    const int64_t items = (int64_t)prm.nqb * prm.B;
-    prm.rank_items = (prm.B >= 2 && prm.B <= fat::kWideRankMaxSeqs && items <= fat::kWideBM) ? (int)items : 0;
-    return fat_host::launch_prefill_wide(prm, dtype == FAT_DTYPE_BF16, causal, grid, stream);
+    rank_wide_items(prm);
+    return fat_host::launch_prefill_wide(prm, dtype == FAT_DTYPE_BF16, causal, false, grid, stream);
   }
   if (dtype == FAT_DTYPE_F16) return launch_prefill_d<fat::F16, PG>(prm, D, causal, kind, grid, stream);
   return launch_prefill_d<fat::BF16, PG>(prm, D, causal, kind, grid, stream);
@@ -1594,6 +1634,62 @@ int64_t paged_stage_rows(const fat_prefill_paged_args* a) {
   return kind == PF_WIDE ? rows : 0;
 }
 
+// Byte offset past the last row of the pool, from a KV head's first row.
+int64_t pool_span(const fat_prefill_paged_args* a, int64_t stride_page, int64_t stride_slot) {
+  return (int64_t)(a->num_pages - 1) * 2 * stride_page + (int64_t)(a->page_size - 1) * 2 * stride_slot +
+         2 * a->head_dim;
+}
+
+// Whether a paged launch that isn't staged runs on the wide kernel, which then
+// reads K, and fp16 V, through the page table: chunks of long contexts, where
+// the queries fill its 512-row blocks (to 80 %), the keys a table may hold are
+// at least four times a chunk, and the grid's rounds over the CUs don't cost
+// what it gains.  Per workgroup it takes 1.76 times the ping-pong kernel's
+// time for twice the rows (packed: 16 x 512 queries over 4096 keys 518 -> 461
+// us in fp16, 9 x 512 over 2048, 288 workgroups, 162 -> 201; over no more
+// than 1024 keys they are level).  bf16 needs V as fp16: a copy of the
+// table's capacity, of at most 8 rows per query (the memory that staging may
+// take), which reads and writes what the kernel reads 16 times or more.
+bool paged_wide(const fat_prefill_paged_args* a) {
+  if (a->head_dim != 128 || (a->dtype != FAT_DTYPE_F16 && a->dtype != FAT_DTYPE_BF16)) return false;
+  if (a->kernel != FAT_KERNEL_AUTO || a->rows != FAT_ROWS_AUTO || a->page_size < 16) return false;
+  if (a->batch <= 0 || a->batch > 65535 || a->total_q <= 0 || a->max_seqlen_q <= 0 || a->num_kv_heads <= 0 ||
+      a->num_heads < a->num_kv_heads || a->max_pages <= 0)
+    return false;
+  // Row offsets from a KV head's first row in 32 bits, 64 KB short of the
+  // offset that stands for rows past the end.
+  auto span_fits = [&](int64_t sp, int64_t ss, int64_t sh) {
+    return sp >= 0 && ss >= 0 && sh >= 0 && ss < (1 << 24) && sp < (1 << 30) && pool_span(a, sp, ss) < 0x7fff0000LL;
+  };
+  if (!span_fits(a->k_stride_page, a->k_stride_slot, a->k_stride_head) ||
+      !span_fits(a->v_stride_page, a->v_stride_slot, a->v_stride_head))
+    return false;
+  const int64_t cap = (int64_t)a->max_pages * a->page_size;
+  if (cap >= (1 << 30) || cap < 4 * (int64_t)a->max_seqlen_q) return false;
+  const int64_t rows = cap * a->batch;
+  if (a->dtype == FAT_DTYPE_BF16 &&
+      (rows > 8 * (int64_t)a->total_q || rows >= 0x7fffffffLL || a->num_kv_heads > 65535 ||
+       2 * cap * a->num_kv_heads * a->head_dim >= 0x7fffffffLL || 2 * a->num_kv_heads * a->head_dim >= (1 << 24)))
+    return false;
+  const int64_t heads = (int64_t)a->batch * a->num_heads;
+  const int64_t nqb = (a->max_seqlen_q + fat::kWideBM - 1) / fat::kWideBM;
+  if (5 * (int64_t)a->total_q < 4 * nqb * fat::kWideBM * a->batch) return false;
+  const int64_t n_pp = (a->max_seqlen_q + fat::kPBM - 1) / fat::kPBM * heads;
+  return nqb * heads <= 0x7fffffff && (nqb * heads + 255) / 256 * 176 <= (n_pp + 255) / 256 * 100;
+}
+
+// Its bf16 V copy: slots for the tile maxima (VpreSeq) and bytes.
+int64_t paged_wide_slots(const fat_prefill_paged_args* a) {
+  const int64_t cap = (int64_t)a->max_pages * a->page_size;
+  return (cap + fat::kVpreRows - 1) / fat::kVpreRows * a->batch;
+}
+size_t paged_wide_v_bytes(const fat_prefill_paged_args* a) {
+  if (a->dtype != FAT_DTYPE_BF16) return 0;
+  const int64_t rows = (int64_t)a->max_pages * a->page_size * a->batch;
+  return vpre_bytes_v16(rows, a->num_kv_heads, a->head_dim) +
+         (size_t)a->num_kv_heads * (paged_wide_slots(a) + a->batch) * sizeof(int32_t);
+}
+
 // Workspace of a staged paged launch (256-byte aligned parts): cu_k [B + 1],
 // the K and V copies [rows, Hkv, D], then the bf16 V pre-pass area.
 struct PagedStageLayout {
@@ -1615,6 +1711,10 @@ extern "C" size_t fat_prefill_paged_workspace_bytes(const fat_prefill_paged_args
   if (!a) return 0;
   const int64_t rows = paged_stage_rows(a);
   return rows > 0 ? paged_stage_layout(a, rows).total : 0;
+}
+
+extern "C" size_t fat_prefill_paged_v_bytes(const fat_prefill_paged_args* a) {
+  return a && paged_stage_rows(a) == 0 && paged_wide(a) ? paged_wide_v_bytes(a) : 0;
 }
 
 extern "C" int fat_prefill_paged(const fat_prefill_paged_args* a, void* stream_ptr) {
@@ -1688,8 +1788,8 @@ extern "C" int fat_prefill_paged(const fat_prefill_paged_args* a, void* stream_p
                         "fat_prefill_paged_workspace_bytes)");
     return FAT_E_UNSUPPORTED;
   }
-  if (a->workspace && ((uintptr_t)a->workspace & 255)) {
-    fat_host::set_error("fat_prefill_paged: workspace must be 256-byte aligned");
+  if (((uintptr_t)a->workspace | (uintptr_t)a->v_workspace) & 255) {
+    fat_host::set_error("fat_prefill_paged: workspaces must be 256-byte aligned");
     return FAT_E_INVALID;
   }
   if (a->max_seqlen_q == 0 || a->total_q == 0) return FAT_OK;  // nothing to compute
@@ -1742,16 +1842,27 @@ extern "C" int fat_prefill_paged(const fat_prefill_paged_args* a, void* stream_p
                              FAT_KERNEL_PREFILL_WIDE, "fat_prefill_paged", stream,
                              L.total > L.vpre ? ws + L.vpre : nullptr, (int)stage_rows, a->total_q);
   }
+  if (stage_rows == 0 && paged_wide(a) && (a->dtype == FAT_DTYPE_F16 || a->v_workspace)) {
+    prm.k_span = (int32_t)pool_span(a, a->k_stride_page, a->k_stride_slot);
+    prm.v_span = (int32_t)pool_span(a, a->v_stride_page, a->v_stride_slot);
+    prm.nqb = (a->max_seqlen_q + fat::kWideBM - 1) / fat::kWideBM;
+    fold_scale(prm, a->softmax_scale);
+    rank_wide_items(prm);
+    if (a->dtype == FAT_DTYPE_BF16) {
+      const int rc = launch_vpre<128, true>(prm, kv_bound * a->batch, (int)paged_wide_slots(a), kv_bound,
+                                            a->v_workspace, stream);
+      if (rc != FAT_OK) return rc;
+    }
+    return fat_host::launch_prefill_wide(prm, a->dtype == FAT_DTYPE_BF16, a->causal != 0, true,
+                                         dim3((unsigned)((int64_t)prm.nqb * prm.B * prm.H)), stream);
+  }
   // One load covers 256 / (D / 8) rows (16 at D128, 32 at D64): with pages at
   // least that long its rows share a page and the page id is wave-uniform.
   bool uniform = P >= 256 / (D / 8);
-  // Byte offset past the last row of the pool, from a KV head's first row:
-  // below 2^31 the uniform loads address the pool as one buffer (PG 3).
-  const int64_t kspan =
-      (int64_t)(a->num_pages - 1) * 2 * a->k_stride_page + (int64_t)(P - 1) * 2 * a->k_stride_slot + 2 * D;
-  const int64_t vspan =
-      (int64_t)(a->num_pages - 1) * 2 * a->v_stride_page + (int64_t)(P - 1) * 2 * a->v_stride_slot + 2 * D;
-  bool off32 = kspan < 0x7fffffffLL && vspan < 0x7fffffffLL;
+  // A pool below 2^31 bytes from a KV head's first row is addressed by the
+  // uniform loads as one buffer (PG 3).
+  bool off32 = pool_span(a, a->k_stride_page, a->k_stride_slot) < 0x7fffffffLL &&
+               pool_span(a, a->v_stride_page, a->v_stride_slot) < 0x7fffffffLL;
   // `rows` forces the per-lane variant (FAT_ROWS_LANE) or the uniform one
   // with 64-bit row addresses (FAT_ROWS_WIDE); all three give identical bits.
   if (a->rows == FAT_ROWS_LANE) uniform = false;

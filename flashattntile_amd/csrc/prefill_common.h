@@ -29,6 +29,9 @@ struct PrefillParams {
   int64_t k_sp, v_sp;   // page strides (elements)
   int32_t pshift;       // log2(page_size)
   int32_t num_pages, max_pages;
+  // Bytes from a KV head's first row to the pool's end (the wide kernel's
+  // paged form: below 2^31 - 2^16).
+  int32_t k_span, v_span;
   // bf16 V converted ahead of the kernel (VPRE instantiations): v points at
   // fp16 values scaled by 2^-v_head_scale[sequence * Hkv + kv head].
   const int32_t* v_head_scale;
@@ -121,10 +124,12 @@ __device__ __forceinline__ void buffer_load_lds16(const i32x4& desc, int voff, i
 
 namespace fat_host {
 // The 8-wave prefill kernel with 64 query rows per wave (prefill_wide.hip)
-// for packed fp16, or packed bf16 whose V was converted to fp16 ahead of the
-// kernel (prm.v / v_head_scale), at head_dim 128.  `grid` counts blocks of
-// fat::kWideBM query rows.
-int launch_prefill_wide(const fat::PrefillParams& prm, bool bf16, bool causal, dim3 grid, hipStream_t stream);
+// for fp16, or bf16 whose V was converted to fp16 ahead of the kernel (prm.v /
+// v_head_scale), at head_dim 128, K and fp16 V packed or (paged) in pages of a
+// power of two >= 16 rows; a converted V is [B max_pages page_size, Hkv, D]
+// then.  `grid` counts blocks of fat::kWideBM query rows.
+int launch_prefill_wide(const fat::PrefillParams& prm, bool bf16, bool causal, bool paged, dim3 grid,
+                        hipStream_t stream);
 // The generic VALU prefill (prefill_generic.hip) for a fat_dtype and a
 // power-of-two head_dim 16..512, packed or paged; `grid` counts blocks of 32
 // query rows.

@@ -86,7 +86,18 @@ struct WideOrder {
 #define FAT_WIDE_LOOK 2
 #endif
 
-// Longest-first order of a packed launch's work items.  Item i = (query
+template <bool PAGED>
+__device__ __forceinline__ int wide_kv_len(const PrefillParams& p, int b) {
+  return PAGED ? min(max(p.lens[b], 0), p.max_pages << p.pshift) : p.cu_k[b + 1] - p.cu_k[b];
+}
+
+// A page id, by a scalar load (the table doesn't change during the launch).
+__device__ __forceinline__ int wide_page(const int32_t* row, int i) {
+  typedef const __attribute__((address_space(4))) int32_t* words;
+  return ((words)(uintptr_t)row)[i];
+}
+
+// Longest-first order of a launch's work items.  Item i = (query
 // block jb = i / B counted from the sequence's end, sequence b = i % B); its
 // causal chain holds kv_len - 512 jb keys (kv_len when not causal).  Items
 // are ordered by chain length (descending), then sequence, then block; items
@@ -95,14 +106,14 @@ struct WideOrder {
 // and the workgroup takes the item of rank `target`, or -1 (no rows: the
 // workgroup exits).  Needs B * nqb <= blockDim.x and a 2 B + 1 int LDS area;
 // every thread of the workgroup calls it.
-template <bool CAUSAL>
+template <bool CAUSAL, bool PAGED>
 __device__ __forceinline__ int wide_ranked_item(const PrefillParams& p, int n, int target, int* s_len) {
   constexpr int BM = kWideBM;
   const int t = threadIdx.x;
   const int B = p.B;
   if (t < B) {
     s_len[2 * t] = p.cu_q[t + 1] - p.cu_q[t];
-    s_len[2 * t + 1] = p.cu_k[t + 1] - p.cu_k[t];
+    s_len[2 * t + 1] = wide_kv_len<PAGED>(p, t);
   }
   if (t == 0) s_len[2 * B] = -1;
   __syncthreads();
@@ -134,7 +145,7 @@ __device__ __forceinline__ int wide_ranked_item(const PrefillParams& p, int n, i
   return s_len[2 * B];
 }
 
-template <typename T, bool CAUSAL>
+template <typename T, bool CAUSAL, bool PAGED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_wide_kernel(const PrefillParams p) {
   constexpr int D = 128;
@@ -156,7 +167,7 @@ void prefill_wide_kernel(const PrefillParams p) {
   int item = blockIdx.x / p.H;
   const int j = blockIdx.x - item * p.H;
   if (p.rank_items > 0) {
-    item = wide_ranked_item<CAUSAL>(p, p.rank_items, item, s_items);
+    item = wide_ranked_item<CAUSAL, PAGED>(p, p.rank_items, item, s_items);
     if (item < 0) return;  // uniform: no item of this rank has rows
   }
   const int jb = item / p.B;
@@ -166,8 +177,8 @@ void prefill_wide_kernel(const PrefillParams p) {
 
   const int q_start = p.cu_q[b];
   const int q_len = p.cu_q[b + 1] - q_start;
-  const int k_start = p.cu_k[b];
-  const int kv_len = p.cu_k[b + 1] - k_start;
+  const int k_start = PAGED ? 0 : p.cu_k[b];
+  const int kv_len = wide_kv_len<PAGED>(p, b);
   if (jb * kWideBM >= q_len) return;  // uniform over the workgroup
   const int r_end = q_len - jb * kWideBM;  // one past the block's last row
 
@@ -200,12 +211,33 @@ void prefill_wide_kernel(const PrefillParams p) {
   const int e_acc = VH ? p.v_head_scale[b * p.Hkv + kvh] : 0;  // bf16: O = acc * 2^e_acc
 
   // This group's stream: K rows (A) or fp16 V rows (B) of the sequence's KV
-  // head, through one buffer descriptor whose range ends with row kv_len - 1.
+  // head, through one buffer descriptor whose range ends with row kv_len - 1,
+  // or, read through the page table (in_pages: PAGED, but for a converted V),
+  // with the pool.
+  const bool in_pages = PAGED && !(VH && grp);
   const int st = grp ? (int)p.v_st : (int)p.k_st;
   const int st2 = 2 * st;
   const int64_t sh = grp ? p.v_sh : p.k_sh;
-  const uint8_t* seq = (grp ? p.v : p.k) + 2 * ((int64_t)k_start * st + (int64_t)kvh * sh);
-  const int rec = (int)min((int64_t)max(kv_len - 1, 0) * st2 + 2 * D, (int64_t)0x7fffffff);
+  const int64_t first_row = PAGED ? (in_pages ? 0 : (int64_t)b * (p.max_pages << p.pshift)) : k_start;
+  const uint8_t* seq = (grp ? p.v : p.k) + 2 * (first_row * st + (int64_t)kvh * sh);
+  const int rec = in_pages ? (grp ? p.v_span : p.k_span)
+                           : (int)min((int64_t)max(kv_len - 1, 0) * st2 + 2 * D, (int64_t)0x7fffffff);
+  // Paged: ids of the pages that hold the next tile's rows 0-15 and 16-31 (one
+  // page or two), fetched a half step or more before that tile's loads.
+  int page0 = 0, page1 = 0;
+  const int32_t* const pt_row = PAGED ? p.pt + (int64_t)b * p.pt_sb : nullptr;
+  auto fetch_pages = [&](int t) __attribute__((always_inline)) {
+    if constexpr (PAGED) {
+      const int key = t * kWideBN;  // <= kv_len + 96: no overflow where kv_len < 2^31 - 96
+      page0 = wide_page(pt_row, min(key >> p.pshift, p.max_pages - 1));
+      page1 = wide_page(pt_row, min((key + 16) >> p.pshift, p.max_pages - 1));
+    }
+  };
+  // Waits for the ids here, in the softmax phase, and not at the first LDS
+  // read of the MFMA phase (scalar loads share its counter).
+  auto hold_pages = [&]() __attribute__((always_inline)) {
+    if constexpr (PAGED) __asm__ volatile("" ::"s"(page0), "s"(page1));
+  };
   // Loads: a tile is 32 rows of `rs` 16-byte slots (rs = 17 for K, 20 for
   // V), 9 (K) or 10 (V) loads of 64 slots; wave wg of the group takes loads
   // wg, wg + 4 and wg + 8.  Slot s holds chunk s % rs of row s / rs; a lane
@@ -227,7 +259,16 @@ void prefill_wide_kernel(const PrefillParams p) {
   // (vmcnt(0)) before each LDS read.  The kernel orders them itself: a
   // wave's own waits (wait_loads), then a workgroup barrier.
   auto issue = [&](int t, int buf) __attribute__((always_inline)) {
-    const int toff = t * kWideBN * st2;
+    // Byte offsets that rows 0-15 and 16-31 of the tile add to r * st2.
+    int off0 = t * kWideBN * st2, off1 = off0;
+    if (PAGED && in_pages) {
+      const int sp2 = 2 * (int)(grp ? p.v_sp : p.k_sp);
+      const int mask = (1 << p.pshift) - 1;
+      const int key = t * kWideBN;
+      off0 = min(max(page0, 0), p.num_pages - 1) * sp2 + (key & mask) * st2;
+      off1 = min(max(page1, 0), p.num_pages - 1) * sp2 + (((key + 16) & mask) - 16) * st2;
+    }
+    const int left = PAGED && in_pages ? kv_len - t * kWideBN : kWideBN;  // rows of the tile that hold keys
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       const int i = wg + 4 * u;
@@ -235,8 +276,12 @@ void prefill_wide_kernel(const PrefillParams p) {
         const int slot = 64 * i + lane;
         const int r = slot / rs;
         const int ch = slot - r * rs;
-        if (ch < 16 && r < kWideBN)
-          buffer_load_lds16(desc, r * st2 + 16 * ch + toff, my_area + buf * tile_bytes + 1024 * i);
+        int voff = r * st2 + 16 * ch + off0;
+        if constexpr (PAGED) {
+          voff += r >= 16 ? off1 - off0 : 0;
+          if (left < kWideBN) voff = r < left ? voff : 0x7ffffff0;  // past the range: zeros
+        }
+        if (ch < 16 && r < kWideBN) buffer_load_lds16(desc, voff, my_area + buf * tile_bytes + 1024 * i);
       }
     }
   };
@@ -252,7 +297,9 @@ void prefill_wide_kernel(const PrefillParams p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[rb][ks] = (*reinterpret_cast<const u32x4*>(qp + 32 * ks) & p.q_and) ^ p.q_xor;
   }
+  fetch_pages(0);
   if (n_tiles > 0) issue(0, 0);
+  fetch_pages(1);
   // Wait until this wave's loads of every tile before the most recent issue
   // have landed (`pending`: that issue's my_loads loads may still be in flight).
   auto wait_loads = [&](bool pending) __attribute__((always_inline)) {
@@ -391,8 +438,10 @@ void prefill_wide_kernel(const PrefillParams p) {
     // 2 n_tiles + 2 barriers.
     auto stage = [&](int t, int buf2) __attribute__((always_inline)) {  // buf2 = (t + 2) % 3
       if (t + 2 < n_tiles) issue(t + 2, buf2);
+      fetch_pages(t + 3);
     };
     auto stage_wait = [&](int t) __attribute__((always_inline)) {
+      hold_pages();
       if (t + 1 < n_tiles) wait_loads(t + 2 < n_tiles);
     };
     if (grp == 0) {  // tile 0 was issued with the Q loads
@@ -463,18 +512,20 @@ void prefill_wide_kernel(const PrefillParams p) {
 
 namespace fat_host {
 
-template <typename T, bool CAUSAL>
-static void launch_wide_c(const fat::PrefillParams& prm, dim3 grid, hipStream_t stream) {
-  hipLaunchKernelGGL((fat::prefill_wide_kernel<T, CAUSAL>), grid, dim3(512), 0, stream, prm);
+template <typename T, bool PAGED>
+static void launch_wide_c(const fat::PrefillParams& prm, bool causal, dim3 grid, hipStream_t stream) {
+  if (causal) hipLaunchKernelGGL((fat::prefill_wide_kernel<T, true, PAGED>), grid, dim3(512), 0, stream, prm);
+  else hipLaunchKernelGGL((fat::prefill_wide_kernel<T, false, PAGED>), grid, dim3(512), 0, stream, prm);
 }
 
-int launch_prefill_wide(const fat::PrefillParams& prm, bool bf16, bool causal, dim3 grid, hipStream_t stream) {
+int launch_prefill_wide(const fat::PrefillParams& prm, bool bf16, bool causal, bool paged, dim3 grid,
+                        hipStream_t stream) {
   if (bf16) {
-    if (causal) launch_wide_c<fat::BF16, true>(prm, grid, stream);
-    else launch_wide_c<fat::BF16, false>(prm, grid, stream);
+    if (paged) launch_wide_c<fat::BF16, true>(prm, causal, grid, stream);
+    else launch_wide_c<fat::BF16, false>(prm, causal, grid, stream);
   } else {
-    if (causal) launch_wide_c<fat::F16, true>(prm, grid, stream);
-    else launch_wide_c<fat::F16, false>(prm, grid, stream);
+    if (paged) launch_wide_c<fat::F16, true>(prm, causal, grid, stream);
+    else launch_wide_c<fat::F16, false>(prm, causal, grid, stream);
   }
   return launch_status("prefill_wide_kernel");
 }

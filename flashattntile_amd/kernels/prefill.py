@@ -371,9 +371,11 @@ def paged_prefill_launch(q: torch.Tensor, cache: PagedKVCache, cu_seqlens_q: tor
 
 
 def _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, out=None, kernel=None, rows=None,
-                 workspace=None):
+                 workspace=None, v_copy=False):
     """The argument block of :func:`paged_prefill_launch`, its output, and
-    the tensors that have to live until the launch is enqueued."""
+    the tensors that have to live until the launch is enqueued.  ``v_copy``:
+    allocate the fp16 copy of V where the library uses one (the launch
+    function, which may be captured, runs without)."""
     if q.stride(-1) != 1 or cache.k_cache.stride(-1) != 1 or cache.v_cache.stride(-1) != 1:
         raise ValueError("q and the cache need a contiguous head_dim axis")
     if out is None:
@@ -391,7 +393,16 @@ def _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, ou
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace = workspace.data_ptr()
-    return a, out, (q, pt, sl, cu, workspace)
+    # bf16 chunks of long contexts read V from an fp16 copy.
+    v16 = None
+    need = _hip.prefill_paged_v_bytes(a) if v_copy else 0
+    if need:
+        try:
+            v16 = torch.empty(need, dtype=torch.uint8, device=q.device)
+            a.v_workspace = v16.data_ptr()
+        except torch.OutOfMemoryError:
+            pass  # the paged kernels need none
+    return a, out, (q, pt, sl, cu, workspace, v16)
 
 
 def paged_prefill_attention(
@@ -459,4 +470,4 @@ def _prepare_paged(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, 
     scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
     q = q if q.stride(-1) == 1 else q.contiguous()
     return _paged_block(q, cache, cu_seqlens_q, int(max_seqlen_q), bool(causal), scale, kernel=cfg["kernel"],
-                        rows=cfg["rows"])
+                        rows=cfg["rows"], v_copy=True)

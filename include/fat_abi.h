@@ -46,7 +46,9 @@
 extern "C" {
 #endif
 
-/* 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
+/* 16: fat_prefill_paged_args.v_workspace and fat_prefill_paged_v_bytes:
+ *     chunks of long contexts on the wide kernel, K read through the pages.
+ * 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
  *     validated call).
  * 14: fat_decode_args.merge_counters and fat_paged_decode_counters_bytes:
  *     split-K decode merges its partitions inside the decode launch.
@@ -65,7 +67,7 @@ extern "C" {
  * 8: fp32 decode, any page size and head_dim 32/256 through the generic
  *    decode kernel (FAT_KERNEL_DECODE_GENERIC); the paged prefill `rows`
  *    field replaces the library's environment overrides. */
-#define FAT_ABI_VERSION 15
+#define FAT_ABI_VERSION 16
 
 /* Element types understood by the kernels. */
 enum fat_dtype {
@@ -296,6 +298,12 @@ typedef struct fat_prefill_args {
  * and runs the packed wide kernel on the copies (`rows` then has no
  * effect); without the workspace it runs the paged kernels.  Same results
  * up to the kernels' rounding (each within the prefill tolerance).
+ * `v_workspace` is optional likewise: NULL, or 256-byte aligned and holding
+ * fat_prefill_paged_v_bytes(args) bytes.  When that is non-zero (bf16,
+ * head_dim 128, chunks that fill the wide kernel's blocks after contexts of
+ * at least three times their length) the launch writes V there as fp16 and
+ * runs the wide kernel, which reads K through the page table; without it, on
+ * the paged kernels.
  */
 typedef struct fat_prefill_paged_args {
   const void* q;
@@ -326,6 +334,7 @@ typedef struct fat_prefill_paged_args {
                      the staging workspace only)                           */
   int32_t rows;   /* FAT_ROWS_AUTO, _WIDE or _LANE                        */
   void* workspace; /* optional, see above                                 */
+  void* v_workspace; /* optional, see above                               */
 } fat_prefill_paged_args;
 
 /*
@@ -466,6 +475,8 @@ int fat_prefill_varlen(const fat_prefill_args* args, void* stream);
  * paged kernels.  Reads only sizes, dtype, causal and kernel; no device
  * access.  No reference counterpart (see fat_prefill_paged). */
 size_t fat_prefill_paged_workspace_bytes(const fat_prefill_paged_args* args);
+/* Bytes of `v_workspace` the launch of `args` uses (0: it runs without). */
+size_t fat_prefill_paged_v_bytes(const fat_prefill_paged_args* args);
 
 /* Enqueue paged (chunked) prefill on `stream`.  Extends
  * flashattn_tile/kernels/prefill.py:236-326 to K/V read through the page
