@@ -212,12 +212,13 @@ def decode_partition(batch: int, num_heads: int, num_kv_heads: int, max_pages: i
 
 
 def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: int, mfma: bool = False,
-                 num_cus: int = MI355X_CUS) -> tuple[int, int | None]:
+                 shared: bool = False, num_cus: int = MI355X_CUS) -> tuple[int, int | None]:
     """``(split_k, waves)`` of a decode launch with ``split_k`` equal
     partitions of every sequence: ``items`` (sequence, head group) pairs, each
     one workgroup when it isn't split, over ``mean_len`` tokens on average and
     ``max_len`` at most, ``item_token_bytes`` of K and V per token and head
-    group, on the MFMA kernel or a VALU one.  Waves None: the library's choice.
+    group, on the MFMA kernel or a VALU one; ``shared``: several head groups
+    read the same lines of K and V.  Waves None: the library's choice.
 
     * As many partitions as fill the CUs once, no shorter than 128 tokens and
       none below 256: a small launch is latency along its longest partition
@@ -232,6 +233,10 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
       1.2 times a CU's share of the tokens and the CU with a workgroup more
       than another has 1.4 times its share: 264 items of 1030-2793 tokens 71.2
       -> 50.1 us, 128 of 1000-7900 with four queries each 66.9 -> 53.7.
+      Grids so split have at least four workgroups per CU, in partitions of
+      512 tokens and more, and so have those whose head groups share lines: 40
+      sequences of 4500 tokens, 8 head groups, int8 at head_dim 64, 85.2 ->
+      65.8 us, 54 of 1950 with 8 head groups per KV head 74 -> 55.
     * Eight waves where a CU has one workgroup, but four on the VALU kernels
       for whole sequences below 1024 tokens (240 items of 609 tokens 17.3 ->
       16.8 us, 33 x 8 of 68 11.4 -> 7.8) and in larger grids, except that the
@@ -256,7 +261,7 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
         while split < min(8, max_len // 256) and items * split > num_cus // 2 \
                 and -(-items * split // num_cus) * num_cus > 1.4 * items * split:
             split += 1
-        if num_cus // 2 < items * split < 4 * num_cus and (split > 1 or items < num_cus):
+        if num_cus // 2 < items * split < 4 * num_cus and (split > 1 or items < num_cus or shared):
             split = max(split, min(-(-4 * num_cus // items), 8, max_len // 512))
     if items * split <= num_cus:
         return split, 4 if not mfma and split == 1 and max_len < 1024 else 8

@@ -262,6 +262,13 @@ void decode_route(const fat_decode_args* a, int kv, DecodeRoute* r) {
                        : (r->mfma ? 32 : (group >= 8 ? 8 : 4));
 }
 
+// KV heads whose rows of one token lie in one 128-byte line of K and of V.
+int line_heads(const fat_decode_args* a, int eb) {
+  const int n = 128 / (eb * a->head_dim);
+  return n > 1 && a->num_kv_heads % n == 0 && a->k_stride_head == a->head_dim && a->v_stride_head == a->head_dim ? n
+                                                                                                              : 1;
+}
+
 // K/V storage of a launch, or -1 where the types don't go together.
 int kv_kind(const fat_decode_args* a) {
   if (a->kv_dtype == a->q_dtype) return fat::KV_SAME;
@@ -498,6 +505,7 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const dim3 grid(a->split_k, a->num_kv_heads * hg_per_kv, a->batch);
   const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+  prm.share = wgs < (1LL << 31) ? hg_per_kv * line_heads(a, eb) : 1;
   const int64_t pages_per_wg =
       a->pages_per_split > 0 ? a->pages_per_split : ((int64_t)a->max_pages + a->split_k - 1) / a->split_k;
   const int bal_rows = a->workspace && a->merge_counters ? balanced_rows(a, kv, route) : 0;

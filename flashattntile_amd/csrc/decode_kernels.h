@@ -290,6 +290,40 @@ __device__ __forceinline__ void merge_rows(const DecodeParams& p, int S, int nro
   if (e1 < n) finish(e1, a1, o1);
 }
 
+// The sequence, head group and partition of this workgroup: its place in the
+// grid, or (share > 1) so that `share` consecutive head groups of a partition
+// run on one XCD and close in time.  Workgroups go to the 8 XCDs in turn by
+// their linear id, so workgroups 8 apart share an L2: 8 units of `share` head
+// groups take each 8 * share ids, what remains of the grid the rest in order.
+// The head groups' loads of the same lines then meet in that L2 instead of
+// each going to memory (40 sequences of 8611 tokens, 16/8 heads, an int8 cache
+// at head_dim 64, 7 partitions 127.6 -> 90.9 us; 54 of 1950, 32/1 heads, bf16,
+// pages of one token, 8 head groups, 5 partitions 87.9 -> 55.8; fp32, 32/1
+// heads, 16 of 1000-4000 60.9 -> 39.1.  A number of partitions that 8 divides
+// did so by chance).
+__device__ __forceinline__ void partition_item(const DecodeParams& p, int& b, int& y, int& split) {
+  b = blockIdx.z;
+  y = blockIdx.y;
+  split = blockIdx.x;
+  if (p.share == 1) return;
+  const unsigned n = (unsigned)p.share, S = gridDim.x, units_y = gridDim.y / n;
+  const unsigned id = split + S * (y + gridDim.y * b);
+  const unsigned whole = units_y * S * gridDim.z / 8 * 8;  // units that go to the XCDs in rounds of 8
+  unsigned unit, k;
+  if (id < whole * n) {
+    const unsigned round = id / (8 * n), r = id - round * 8 * n;
+    unit = round * 8 + r % 8;
+    k = r / 8;
+  } else {
+    unit = whole + (id - whole * n) / n;
+    k = (id - whole * n) % n;
+  }
+  const unsigned row = unit / S;
+  split = unit - row * S;
+  b = row / units_y;
+  y = (row - b * units_y) * n + k;
+}
+
 // Split-K merge inside the decode launch (p.counters set).  Every thread has
 // written its part of this workgroup's (acc, m, l) rows with device-scope
 // stores (ws_store, global_store ... sc1: written through to the level all
@@ -305,14 +339,14 @@ __device__ __forceinline__ void merge_rows(const DecodeParams& p, int S, int nro
 // (buffer_wbl2), which measured 7-16 % slower on 8-sequence split
 // launches.  No workgroup waits for another.
 template <typename QT, int D, typename RowOf>
-__device__ __forceinline__ void merge_in_launch(const DecodeParams& p, int S, int nrows, RowOf row_of) {
+__device__ __forceinline__ void merge_in_launch(const DecodeParams& p, int S, int item, int nrows, RowOf row_of) {
   __shared__ int s_last;
   __shared__ float s_f[32 * 16];  // merge weights of up to 32 rows x 16 partitions
   __shared__ float s_l[32];
   __atomic_signal_fence(__ATOMIC_SEQ_CST);  // keep the row stores before the wait
   __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): this wave's row stores are complete
   __syncthreads();
-  int* const cnt = p.counters + (blockIdx.z * gridDim.y + blockIdx.y);
+  int* const cnt = p.counters + item;
   if (threadIdx.x == 0) {
     const int prev = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     s_last = prev == S - 1;
@@ -1041,7 +1075,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
       bal_merge<QT, D, NW * 64>(p, item, w_first, n_parts, nvalid,
                                 [&](int j) { return (int64_t)b * p.o_sb + (int64_t)(head0 + j) * p.o_sh; }, s_f, s_mm);
   } else if (S > 1 && p.counters) {
-    merge_in_launch<QT, D>(p, S, nvalid, [&](int j, int64_t& bh, int64_t& o) {
+    merge_in_launch<QT, D>(p, S, b * gridDim.y + y, nvalid, [&](int j, int64_t& bh, int64_t& o) {
       const int h = head0 + j;
       bh = (int64_t)b * p.H + h;
       o = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
@@ -1056,7 +1090,9 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
                                   segment(q, b, y, 0, 1, t_begin, t_end, slot, item, w_first, n);
                                 });
   } else {
-    segment(p, blockIdx.z, blockIdx.y, blockIdx.x, gridDim.x, 0, 0, 0, 0, 0, 0);
+    int b, y, split;
+    partition_item(p, b, y, split);
+    segment(p, b, y, split, gridDim.x, 0, 0, 0, 0, 0, 0);
   }
 }
 
@@ -1429,7 +1465,7 @@ void paged_decode_mfma_kernel(const DecodeParams p) {
       }, s_f, s_f + kBalRows * 64);
     }
   } else if (S > 1 && p.counters) {
-    merge_in_launch<QT, D>(p, S, nvalid, [&](int j, int64_t& bh, int64_t& o) {
+    merge_in_launch<QT, D>(p, S, b * gridDim.y + y, nvalid, [&](int j, int64_t& bh, int64_t& o) {
       const int rr = row_base + j;
       const int tt = rr / p.group;
       const int h = kvh * p.group + (rr - tt * p.group);
@@ -1446,7 +1482,9 @@ void paged_decode_mfma_kernel(const DecodeParams p) {
                                   segment(q, b, y, 0, 1, t_begin, t_end, slot, item, w_first, n);
                                 });
   } else {
-    segment(p, blockIdx.z, blockIdx.y, blockIdx.x, gridDim.x, 0, 0, 0, 0, 0, 0);
+    int b, y, split;
+    partition_item(p, b, y, split);
+    segment(p, b, y, split, gridDim.x, 0, 0, 0, 0, 0, 0);
   }
 }
 

@@ -34,8 +34,12 @@ struct DecodeParams {
   uint32_t invP;  // floor(2^32 / page_size), page_size > 1
   int32_t pps_fixed;  // pages per partition, 0 = ceil(np / split_k)
   float scale_log2;  // softmax_scale * log2(e)
+  // Consecutive head groups that read the same lines of K and V (more than one
+  // per KV head, or heads whose rows are parts of one line): partition_item
+  // runs them on one XCD.  1: the grid's own order.
+  int32_t share;
   // Split-K merge inside the decode launch: one counter per (sequence, head
-  // group) = blockIdx.z * gridDim.y + blockIdx.y, zero between launches;
+  // group) = sequence * gridDim.y + head group, zero between launches;
   // nullptr: a second kernel merges.  smax: the merge's unrolled partition
   // count (a power of two >= split_k, at most 16).
   int32_t* counters;

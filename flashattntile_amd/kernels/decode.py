@@ -112,11 +112,15 @@ def resolve_decode_config(q: torch.Tensor, cache: PagedKVCache, max_len: int, to
     return _resolve_config(config, q, cache, max_len, total_pages, q_len)
 
 
-def _work_items(q: torch.Tensor, cache: PagedKVCache, kernel: str | None, q_len: int) -> tuple[int, int, bool, bool]:
-    """``(rows, items, mfma, balances)`` of a decode launch: the (query head,
+def _work_items(q: torch.Tensor, cache: PagedKVCache, kernel: str | None, q_len: int) \
+        -> tuple[int, int, bool, bool, bool]:
+    """``(rows, items, mfma, shared, balances)`` of a decode launch: the (query head,
     token) rows of one workgroup, the (sequence, head group) pairs of the
     batch, whether the library takes the MFMA kernel (``fat_paged_decode``),
-    and whether the kernel that it takes has a balanced form."""
+    whether head groups share lines of K and V, which partitions keep on one
+    XCD and balanced runs do not (27 sequences of 8167-20782 tokens on an int8
+    cache at head_dim 64: 97 us in five partitions, 132 balanced), and whether
+    the launch has a balanced form that gains."""
     group = int(q.shape[-2]) // cache.num_kv_heads
     rows = group * q_len
     quantized = cache.k_cache.dtype in _QUANT_DTYPES
@@ -132,7 +136,11 @@ def _work_items(q: torch.Tensor, cache: PagedKVCache, kernel: str | None, q_len:
         balances = d >= (64 if quantized else 32) and d <= (256 if quantized else 128)
     if kernel == "generic":
         per_wg, balances = 8, False
-    return min(rows, per_wg), int(q.shape[0]) * cache.num_kv_heads * -(-rows // per_wg), per_wg == 32, balances
+    per_line = 128 // (cache.k_cache.element_size() * d)
+    shared = rows > per_wg or (per_line > 1 and cache.num_kv_heads % per_line == 0 and
+                               cache.k_cache.stride(2) == cache.v_cache.stride(2) == d)
+    items = int(q.shape[0]) * cache.num_kv_heads * -(-rows // per_wg)
+    return min(rows, per_wg), items, per_wg == 32, shared, balances and not shared
 
 
 def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: int, total_pages: int,
@@ -144,7 +152,7 @@ def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: i
         batch, heads, hkv, page = int(q.shape[0]), int(q.shape[-2]), cache.num_kv_heads, cache.page_size
         max_pages = -(-max_len // page)
         k = cache.k_cache
-        rows, items, mfma, balances = _work_items(q, cache, resolved["kernel"], q_len)
+        rows, items, mfma, shared, balances = _work_items(q, cache, resolved["kernel"], q_len)
         mean_len = min(max_len, total_pages * page / max(1, batch))
         token_bytes = 2 * cache.head_dim * k.element_size()
         if resolved["balanced"] is None and resolved["pages_per_split"] is None and waves in (None, 4) \
@@ -164,7 +172,7 @@ def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: i
             if resolved["num_warps"] is None and is_ragged(batch, max_pages, total_pages):
                 resolved["num_warps"] = 4
         else:
-            resolved["split_k"], chosen = decode_split(items, max_len, mean_len, token_bytes, mfma)
+            resolved["split_k"], chosen = decode_split(items, max_len, mean_len, token_bytes, mfma, shared)
             resolved["pages_per_split"] = 0
             if resolved["num_warps"] is None:
                 resolved["num_warps"] = chosen
