@@ -1015,7 +1015,8 @@ def all_configs(args, device):
 # passes ran on; the bench line carries its figures only while the files
 # still hash to that digest (otherwise the kernel changed since).
 PROFILE_SOURCES = {
-    "decode": ["flashattntile_amd/csrc/decode.hip", "flashattntile_amd/csrc/decode_params.h",
+    "decode": ["flashattntile_amd/csrc/decode.hip", "flashattntile_amd/csrc/decode_kernels.h",
+               "flashattntile_amd/csrc/decode_balanced.hip", "flashattntile_amd/csrc/decode_params.h",
                "flashattntile_amd/csrc/fat_common.h"],
     "prefill": ["flashattntile_amd/csrc/prefill.hip", "flashattntile_amd/csrc/prefill_wide.hip",
                 "flashattntile_amd/csrc/prefill_common.h", "flashattntile_amd/csrc/fat_common.h"],
