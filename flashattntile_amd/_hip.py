@@ -192,6 +192,7 @@ class PrefillPagedArgs(ctypes.Structure):
         ("rows", _c_i32),
         ("workspace", _c_vp),
         ("v_workspace", _c_vp),
+        ("total_k", _c_i64),
     ]
 
 

@@ -1642,12 +1642,13 @@ int64_t pool_span(const fat_prefill_paged_args* a, int64_t stride_page, int64_t 
 
 // Whether a paged launch that isn't staged runs on the wide kernel, which then
 // reads K, and fp16 V, through the page table: chunks of long contexts, where
-// the queries fill its 512-row blocks (to 80 %), the keys a table may hold are
-// at least four times a chunk, and the grid's rounds over the CUs don't cost
+// the queries fill its 512-row blocks (to 80 %), the caller says that the batch
+// holds at least four times as many keys (total_k), and the grid's rounds over the CUs don't cost
 // what it gains.  Per workgroup it takes 1.76 times the ping-pong kernel's
 // time for twice the rows (packed: 16 x 512 queries over 4096 keys 518 -> 461
-// us in fp16, 9 x 512 over 2048, 288 workgroups, 162 -> 201; over no more
-// than 1024 keys they are level).  bf16 needs V as fp16: a copy of the
+// us in fp16, 9 x 512 over 2048, 288 workgroups, 162 -> 201; paged calls over
+// 2048 keys 268 -> 262 in fp16 and 293 -> 290 in bf16, over 1024 147 -> 147 and
+// 160 -> 168, 32 first chunks 162 -> 167 and 179 -> 205).  bf16 needs V as fp16: a copy of the
 // table's capacity, of at most 8 rows per query (the memory that staging may
 // take), which reads and writes what the kernel reads 16 times or more.
 bool paged_wide(const fat_prefill_paged_args* a) {
@@ -1665,7 +1666,7 @@ bool paged_wide(const fat_prefill_paged_args* a) {
       !span_fits(a->v_stride_page, a->v_stride_slot, a->v_stride_head))
     return false;
   const int64_t cap = (int64_t)a->max_pages * a->page_size;
-  if (cap >= (1 << 30) || cap < 4 * (int64_t)a->max_seqlen_q) return false;
+  if (cap >= (1 << 30) || a->total_k < 4 * (int64_t)a->total_q) return false;
   const int64_t rows = cap * a->batch;
   if (a->dtype == FAT_DTYPE_BF16 &&
       (rows > 8 * (int64_t)a->total_q || rows >= 0x7fffffffLL || a->num_kv_heads > 65535 ||

@@ -371,11 +371,9 @@ def paged_prefill_launch(q: torch.Tensor, cache: PagedKVCache, cu_seqlens_q: tor
 
 
 def _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, out=None, kernel=None, rows=None,
-                 workspace=None, v_copy=False):
+                 workspace=None):
     """The argument block of :func:`paged_prefill_launch`, its output, and
-    the tensors that have to live until the launch is enqueued.  ``v_copy``:
-    allocate the fp16 copy of V where the library uses one (the launch
-    function, which may be captured, runs without)."""
+    the tensors that have to live until the launch is enqueued."""
     if q.stride(-1) != 1 or cache.k_cache.stride(-1) != 1 or cache.v_cache.stride(-1) != 1:
         raise ValueError("q and the cache need a contiguous head_dim axis")
     if out is None:
@@ -393,16 +391,7 @@ def _paged_block(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, ou
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
         a.workspace = workspace.data_ptr()
-    # bf16 chunks of long contexts read V from an fp16 copy.
-    v16 = None
-    need = _hip.prefill_paged_v_bytes(a) if v_copy else 0
-    if need:
-        try:
-            v16 = torch.empty(need, dtype=torch.uint8, device=q.device)
-            a.v_workspace = v16.data_ptr()
-        except torch.OutOfMemoryError:
-            pass  # the paged kernels need none
-    return a, out, (q, pt, sl, cu, workspace, v16)
+    return a, out, (q, pt, sl, cu, workspace)
 
 
 def paged_prefill_attention(
@@ -425,6 +414,7 @@ def paged_prefill_attention(
     """
     _check_paged_shapes(q, cache, cu_seqlens_q)
     check = block = error = None
+    total_k = 0  # not known
     if q.is_cuda and cache.page_table.numel() and _hip.is_loaded():
         # as in prefill_attention: the check runs while the launch is prepared
         stream = _hip.current_stream_handle(q.device)
@@ -438,7 +428,7 @@ def paged_prefill_attention(
         except Exception as exc:
             error = exc
         r = check.wait()
-        flags, first = r[7], r[10]
+        flags, first, total_k = r[7], r[10], r[2] * cache.page_size
         stats = [r[3], r[4], flags & 1, r[8], flags & 4, r[0], r[1], r[12], r[13], first >= 0, first, r[11]]
     else:
         stats = _paged_stats(cache, cu_seqlens_q)
@@ -453,6 +443,16 @@ def paged_prefill_attention(
         block = _prepare_paged(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, config)
         stream = _hip.current_stream_handle(q.device)
     a, out, _keep = block
+    # Chunks of long contexts run on the wide kernel, bf16 ones with an fp16
+    # copy of V; where that can't be had, the paged kernels need none.
+    a.total_k = total_k
+    need = _hip.prefill_paged_v_bytes(a)
+    if need:
+        try:
+            v16 = torch.empty(need, dtype=torch.uint8, device=q.device)
+            a.v_workspace = v16.data_ptr()
+        except torch.OutOfMemoryError:
+            pass
     _hip.prefill_paged_with_args(a, stream)
     return out
 
@@ -470,4 +470,4 @@ def _prepare_paged(q, cache, cu_seqlens_q, max_seqlen_q, causal, softmax_scale, 
     scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
     q = q if q.stride(-1) == 1 else q.contiguous()
     return _paged_block(q, cache, cu_seqlens_q, int(max_seqlen_q), bool(causal), scale, kernel=cfg["kernel"],
-                        rows=cfg["rows"], v_copy=True)
+                        rows=cfg["rows"])

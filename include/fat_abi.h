@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-/* 16: fat_prefill_paged_args.v_workspace and fat_prefill_paged_v_bytes:
+/* 16: fat_prefill_paged_args.v_workspace, .total_k and fat_prefill_paged_v_bytes:
  *     chunks of long contexts on the wide kernel, K read through the pages.
  * 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
  *     validated call).
@@ -300,8 +300,8 @@ typedef struct fat_prefill_args {
  * up to the kernels' rounding (each within the prefill tolerance).
  * `v_workspace` is optional likewise: NULL, or 256-byte aligned and holding
  * fat_prefill_paged_v_bytes(args) bytes.  When that is non-zero (bf16,
- * head_dim 128, chunks that fill the wide kernel's blocks after contexts of
- * at least three times their length) the launch writes V there as fp16 and
+ * head_dim 128, chunks that fill the wide kernel's blocks, total_k at least
+ * four times total_q) the launch writes V there as fp16 and
  * runs the wide kernel, which reads K through the page table; without it, on
  * the paged kernels.
  */
@@ -335,6 +335,8 @@ typedef struct fat_prefill_paged_args {
   int32_t rows;   /* FAT_ROWS_AUTO, _WIDE or _LANE                        */
   void* workspace; /* optional, see above                                 */
   void* v_workspace; /* optional, see above                               */
+  int64_t total_k; /* the batch's seq_lens summed, rounded up to pages or not,
+                      where the caller knows it; 0: the paged kernels alone  */
 } fat_prefill_paged_args;
 
 /*

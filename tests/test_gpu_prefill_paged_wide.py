@@ -21,9 +21,9 @@ from test_gpu_prefill_paged import _case, _ref32
 pytestmark = pytest.mark.gpu
 
 # (kv_len, q_len): 160 blocks of the wide kernel at 32 heads, 320 of the ping-pong kernel's.
-SHORT = [(2048, 512), (2047, 512), (430, 430), (1999, 512), (701, 500)]
+SHORT = [(3840, 512), (3701, 512), (430, 430), (1999, 512), (701, 500)]
 # More sequences than the kernel ranks, two blocks per sequence, the first of them partly filled.
-LONG = [(4000 - 97 * i, 1024 - 11 * i) for i in range(17)]
+LONG = [(6000 - 97 * i, 1024 - 11 * i) for i in range(17)]
 
 
 def _launch(lens, h, hk, P, dtype, seed):
@@ -35,6 +35,8 @@ def _launch(lens, h, hk, P, dtype, seed):
 def _v_bytes(q, cache, cu, mq, causal, P):
     a = _hip.prefill_paged_args(q, cache.k_cache, cache.v_cache, cache.page_table, cache.seq_lens, cu, q, P, mq,
                                 causal, 128 ** -0.5)
+    assert _hip.prefill_paged_v_bytes(a) == 0  # the contexts' lengths are not known: the paged kernels
+    a.total_k = int(cache.seq_lens.sum())
     return _hip.prefill_paged_v_bytes(a)
 
 
