@@ -108,7 +108,7 @@ def _check_shapes(q, k, v, cu_seqlens_q, cu_seqlens_k) -> None:
 
 
 def _varlen_stats(cu_seqlens_q, cu_seqlens_k) -> list[int]:
-    """What ``_judge_varlen`` checks, by torch reductions and one copy (CPU
+    """What ``_assess_varlen`` checks, by torch reductions and one copy (CPU
     tensors; ROCm tensors take the check kernel)."""
     cq = cu_seqlens_q.to(torch.int64)
     ck = cu_seqlens_k.to(torch.int64)
@@ -125,7 +125,7 @@ def _varlen_stats(cu_seqlens_q, cu_seqlens_k) -> list[int]:
     return [int(x) for x in stats]
 
 
-def _judge_varlen(stats, q, k, causal) -> tuple[int, int]:
+def _assess_varlen(stats, q, k, causal) -> tuple[int, int]:
     """The device-side checks of ``prefill.py:194-233`` on their numbers.
 
     Returns the longest query and key sequence lengths."""
@@ -236,7 +236,7 @@ def prefill_attention(
         stats = [r[3], r[5], r[4], r[6], flags & 1, flags & 2, flags & 4, r[8], r[9], first >= 0, first, r[11]]
     else:
         stats = _varlen_stats(cu_seqlens_q, cu_seqlens_k)
-    longest_q, longest_k = _judge_varlen(stats, q, k, causal)
+    longest_q, longest_k = _assess_varlen(stats, q, k, causal)
     if max_seqlen_q <= 0:
         raise ValueError(f"max_seqlen_q must be positive, got {max_seqlen_q}")
     if max_seqlen_k <= 0:
@@ -302,7 +302,7 @@ def _check_paged_shapes(q, cache: PagedKVCache, cu_seqlens_q) -> None:
 
 
 def _paged_stats(cache: PagedKVCache, cu_seqlens_q) -> list[int]:
-    """What ``_judge_paged`` checks, by torch reductions and one copy (CPU
+    """What ``_assess_paged`` checks, by torch reductions and one copy (CPU
     tensors; ROCm tensors take the check kernel)."""
     dev = cu_seqlens_q.device
     cq = cu_seqlens_q.to(torch.int64)
@@ -324,7 +324,7 @@ def _paged_stats(cache: PagedKVCache, cu_seqlens_q) -> list[int]:
     return [int(x) for x in stats]
 
 
-def _judge_paged(stats, q, cache: PagedKVCache, causal) -> int:
+def _assess_paged(stats, q, cache: PagedKVCache, causal) -> int:
     """The device-side checks (cu_seqlens_q monotone and ending at
     q.shape[0]; lengths within the table; used pages inside the pool; kv_len
     >= q_len when causal) on their numbers.  Returns the longest query
@@ -432,7 +432,7 @@ def paged_prefill_attention(
         stats = [r[3], r[4], flags & 1, r[8], flags & 4, r[0], r[1], r[12], r[13], first >= 0, first, r[11]]
     else:
         stats = _paged_stats(cache, cu_seqlens_q)
-    longest_q = _judge_paged(stats, q, cache, causal)
+    longest_q = _assess_paged(stats, q, cache, causal)
     if max_seqlen_q <= 0:
         raise ValueError(f"max_seqlen_q must be positive, got {max_seqlen_q}")
     if max_seqlen_q < longest_q:

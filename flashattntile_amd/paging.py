@@ -159,10 +159,10 @@ def validate_cache(cache: PagedKVCache, *, check_pages: bool = True) -> tuple[in
     ``(min_len, max_len)`` so callers need no further synchronisation.
     """
     _check_layout(cache)
-    return _judge_cache(cache, cache_stats(cache), check_pages)
+    return _assess_cache(cache, cache_stats(cache), check_pages)
 
 
-def _judge_cache(cache: PagedKVCache, stats: tuple[int, ...], check_pages: bool = True) -> tuple[int, int]:
+def _assess_cache(cache: PagedKVCache, stats: tuple[int, ...], check_pages: bool = True) -> tuple[int, int]:
     """The device-side checks of :func:`validate_cache` on their numbers."""
     min_len, max_len, lo, hi = stats
     _require(min_len >= 0, "seq_lens must be non-negative")

@@ -26,7 +26,7 @@ from dataclasses import dataclass
 
 import torch
 
-from .paging import PagedKVCache, _check_layout, _judge_cache, cache_stats
+from .paging import PagedKVCache, _check_layout, _assess_cache, cache_stats
 
 __all__ = [
     "FP8_DTYPE",
@@ -213,11 +213,11 @@ def quantize_cache(cache: PagedKVCache, mode: str = "auto") -> tuple[PagedKVCach
         except Exception as exc:  # raised after the validation's own errors
             error = exc
         r = check.wait()
-        _judge_cache(cache, (r[0], r[1], r[12], r[13]))
+        _assess_cache(cache, (r[0], r[1], r[12], r[13]))
         if error is not None:
             raise error
     else:
-        _judge_cache(cache, cache_stats(cache))
+        _assess_cache(cache, cache_stats(cache))
         done = _quantize_kv_pages(cache.k_cache, cache.v_cache, mode)
     qk, qv, sk, sv, info = _with_scale_range(*done)
     quantized = PagedKVCache(k_cache=qk, v_cache=qv, page_table=cache.page_table,
