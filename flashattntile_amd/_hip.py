@@ -21,7 +21,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libfat_hip.so"
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 # enum fat_dtype
 DT_F16 = 0
@@ -117,6 +117,7 @@ class DecodeArgs(ctypes.Structure):
         ("kernel", _c_i32),
         ("merge_counters", _c_vp),
         ("balanced", _c_i32),
+        ("workspace_bytes", _c_i64),
     ]
 
 
@@ -622,7 +623,7 @@ def decode_args(
     a.page_table = _ptr(page_table)
     a.seq_lens = _ptr(seq_lens)
     a.out = _ptr(out)
-    a.workspace = _ptr(workspace)
+    set_workspace(a, workspace)
     if multi:
         a.q_stride_b, a.q_stride_t, a.q_stride_h = q.stride(0), q.stride(1), q.stride(2)
         a.out_stride_t = out.stride(1)
@@ -651,6 +652,13 @@ def decode_args(
     a.kernel = int(kernel)
     a.merge_counters = _ptr(counters)
     return a
+
+
+def set_workspace(a: DecodeArgs, workspace: torch.Tensor | None) -> None:
+    """Point ``a`` at ``workspace`` and state its size (a launch that needs
+    more is refused)."""
+    a.workspace = _ptr(workspace)
+    a.workspace_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
 
 
 def decode_with_args(a: DecodeArgs, stream: int) -> None:

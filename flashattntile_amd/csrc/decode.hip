@@ -298,6 +298,11 @@ int balanced_rows(const fat_decode_args* a, int kv, const DecodeRoute& r) {
 // 2-14 % slower on the others).
 int balanced_groups(const fat_decode_args* a) { return a->balanced > 1 ? a->balanced : 512; }
 
+// Its workspace: two partial rows (acc, m, l) per row and workgroup.
+size_t balanced_bytes(const fat_decode_args* a, int rows) {
+  return (size_t)balanced_groups(a) * 2 * rows * (a->head_dim + 2) * sizeof(float);
+}
+
 }  // namespace
 
 extern "C" size_t fat_paged_decode_balanced_workspace_bytes(const fat_decode_args* a) {
@@ -309,7 +314,7 @@ extern "C" size_t fat_paged_decode_balanced_workspace_bytes(const fat_decode_arg
   DecodeRoute r;
   decode_route(a, kv, &r);
   const int rows = balanced_rows(a, kv, r);
-  return rows ? (size_t)balanced_groups(a) * 2 * rows * (a->head_dim + 2) * sizeof(float) : 0;
+  return rows ? balanced_bytes(a, rows) : 0;
 }
 
 extern "C" size_t fat_paged_decode_workspace_bytes(int32_t batch, int32_t num_heads, int32_t head_dim,
@@ -389,6 +394,10 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   }
   if ((uintptr_t)a->merge_counters & 3) {
     fat_host::set_error("fat_paged_decode: merge_counters must be 4-byte aligned");
+    return FAT_E_INVALID;
+  }
+  if (a->workspace_bytes < 0) {
+    fat_host::set_error("fat_paged_decode: workspace_bytes must be >= 0, got %lld", (long long)a->workspace_bytes);
     return FAT_E_INVALID;
   }
   if (a->q_len < 0 || a->q_len > 64) {
@@ -509,6 +518,13 @@ extern "C" int fat_paged_decode(const fat_decode_args* a, void* stream_ptr) {
   const int64_t pages_per_wg =
       a->pages_per_split > 0 ? a->pages_per_split : ((int64_t)a->max_pages + a->split_k - 1) / a->split_k;
   const int bal_rows = a->workspace && a->merge_counters ? balanced_rows(a, kv, route) : 0;
+  const size_t ws_need = bal_rows ? balanced_bytes(a, bal_rows)
+                                  : fat_paged_decode_workspace_bytes(a->batch * T, a->num_heads, D, a->split_k);
+  if (a->workspace_bytes > 0 && ws_need > (size_t)a->workspace_bytes) {
+    fat_host::set_error("fat_paged_decode: this launch needs %zu bytes of workspace, the caller's holds %lld", ws_need,
+                        (long long)a->workspace_bytes);
+    return FAT_E_INVALID;
+  }
   if (bal_rows) {
     const int groups = balanced_groups(a);
     prm.counters = a->merge_counters;
@@ -630,6 +646,7 @@ extern "C" int fat_paged_decode_noalloc(const fat_decode_args* a, void* stream) 
   }
   fat_decode_args b = *a;
   b.workspace = need ? g_scratch_ptr[dev] : nullptr;
+  b.workspace_bytes = (int64_t)kScratchBytes;
   b.merge_counters = nullptr;  // a second kernel merges: no state outside the scratch array
   const int rc = fat_paged_decode(&b, stream);
   if (rc != FAT_OK) {

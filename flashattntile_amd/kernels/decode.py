@@ -362,7 +362,7 @@ def _launch_block(a, q, split_k, workspace=None, waves_per_group=None, pages_per
     if counters is not None and counters.numel() * counters.element_size() < 4 * rows * q.shape[-2]:
         raise ValueError("paged_decode_launch: counters smaller than decode_counters_bytes(rows, num_heads)")
     a.split_k = int(split_k)
-    a.workspace = None if workspace is None else workspace.data_ptr()
+    _hip.set_workspace(a, workspace)
     a.waves_per_group = waves_per_group or 0
     a.pages_per_split = int(pages_per_split)
     a.kernel = _KERNEL_CODES[kernel]
@@ -384,6 +384,15 @@ def _balance(a, cfg) -> int:
     return need
 
 
+def _plan_workspace_bytes(a, cfg) -> int:
+    """Set up the block ``a`` of a prepared launch as :func:`_balance` does and
+    return the workspace bytes that cover each of its runs: a run whose query
+    isn't 16-byte aligned can go to the generic kernel, which has no balanced
+    form, and then takes ``a``'s partitions (0: neither form uses any)."""
+    rows = a.batch * max(1, a.q_len)
+    return max(_balance(a, cfg), _hip.decode_workspace_bytes(rows, a.num_heads, a.head_dim, cfg["split_k"]))
+
+
 def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     """Launch with the resolved partitions, from the prepared block if there
     is one."""
@@ -394,7 +403,7 @@ def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     need = _balance(a, cfg)
     if need:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-        a.workspace = workspace.data_ptr()
+        _hip.set_workspace(a, workspace)
         a.merge_counters = merge_counters(q, 2).data_ptr()
         _hip.decode_with_args(a, _hip.current_stream_handle(q.device))
         del keep
@@ -583,22 +592,18 @@ class DecodeLaunch:
             raise ValueError("DecodeLaunch: page_table rows and seq_lens must be contiguous")
         self.config = cfg
         self.softmax_scale = float(softmax_scale) if softmax_scale is not None else q.shape[-1] ** -0.5
-        rows = q.shape[0] * q_len
         self._args = _hip.decode_args(q, cache.k_cache, cache.v_cache, cache.page_table, cache.seq_lens, q,
                                       cache.page_size, self.softmax_scale, cfg["split_k"], k_scale=k_scale,
                                       v_scale=v_scale, waves_per_group=cfg["num_warps"] or 0,
                                       pages_per_split=cfg["pages_per_split"], kernel=_KERNEL_CODES[cfg["kernel"]])
-        need = _balance(self._args, cfg)
-        merged = bool(need) or cfg["split_k"] > 1
-        if not need:
-            need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], cfg["split_k"])
-        self.workspace = torch.empty(max(1, need), dtype=torch.uint8, device=q.device) if need else None
+        need = _plan_workspace_bytes(self._args, cfg)
+        self.workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
         # Zeroed merge counters of this launch (each run leaves them zero):
         # the decode kernel merges its partitions itself.  Runs of one
         # DecodeLaunch share them, as they share the workspace.
-        self.counters = (torch.zeros(_hip.decode_counters_bytes(rows, q.shape[-2]) // 4, dtype=torch.int32,
-                                     device=q.device) if merged else None)
-        self._args.workspace = None if self.workspace is None else self.workspace.data_ptr()
+        self.counters = (torch.zeros(_hip.decode_counters_bytes(q.shape[0] * q_len, q.shape[-2]) // 4,
+                                     dtype=torch.int32, device=q.device) if need else None)
+        _hip.set_workspace(self._args, self.workspace)
         self._args.merge_counters = None if self.counters is None else self.counters.data_ptr()
         self._keep = (cache, k_scale, v_scale)  # the argument block points into these
         self._shape, self._dtype = tuple(q.shape), q.dtype

@@ -46,7 +46,8 @@
 extern "C" {
 #endif
 
-/* 16: fat_prefill_paged_args.v_workspace, .total_k and fat_prefill_paged_v_bytes:
+/* 17: fat_decode_args.workspace_bytes.
+ * 16: fat_prefill_paged_args.v_workspace, .total_k and fat_prefill_paged_v_bytes:
  *     chunks of long contexts on the wide kernel, K read through the pages.
  * 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
  *     validated call).
@@ -67,7 +68,7 @@ extern "C" {
  * 8: fp32 decode, any page size and head_dim 32/256 through the generic
  *    decode kernel (FAT_KERNEL_DECODE_GENERIC); the paged prefill `rows`
  *    field replaces the library's environment overrides. */
-#define FAT_ABI_VERSION 16
+#define FAT_ABI_VERSION 17
 
 /* Element types understood by the kernels. */
 enum fat_dtype {
@@ -221,6 +222,14 @@ typedef struct fat_decode_args {
    * workgroups, else that many (to 4096).  Where it hasn't, split_k
    * partitions as with 0. */
   int32_t balanced;
+  /* Bytes that `workspace` holds: a launch that would write more is refused
+   * (FAT_E_INVALID, nothing runs).  0: not stated, the caller vouches for the
+   * size.  Which form a launch takes, and so what it writes, depends on the
+   * query's address too: a block with `balanced` set whose queries are not
+   * all 16-byte aligned needs the larger of
+   * fat_paged_decode_balanced_workspace_bytes (of an aligned query) and
+   * fat_paged_decode_workspace_bytes. */
+  int64_t workspace_bytes;
 } fat_decode_args;
 
 /*

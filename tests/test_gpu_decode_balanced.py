@@ -132,3 +132,24 @@ def test_balanced_falls_back(heads):
         out = paged_decode_attention(q, cache, config=cfg)
         torch.cuda.synchronize()
         _check(out, ref, f"fallback H{h}/{hk} {cfg}")
+
+
+@pytest.mark.parametrize("dtype,d,P", [(torch.float16, 128, 1), (torch.bfloat16, 64, 3), (torch.float32, 64, 16)])
+def test_balanced_plan_takes_unaligned_queries(dtype, d, P):
+    """A prepared balanced launch run with contiguous queries that aren't
+    16-byte aligned: the generic kernel, in the plan's workspace."""
+    k, v, pt, sl = make_paged(LENS, 2, d, P, dtype, seed=31, device=DEV)
+    cache = PagedKVCache(k, v, pt, sl, P)
+    q = make_query(len(LENS), 8, d, dtype, seed=32, device=DEV)
+    ref = _oracle(q, k, v, pt, sl)
+    plan = DecodeLaunch(q, cache, config={"balanced": 1, "split_k": 11})
+    assert plan._args.balanced
+    flat = torch.empty(q.numel() + 16, dtype=dtype, device=DEV)
+    for offset in (0, 1, 3, 0):
+        label = f"balanced plan, query at {offset} {dtype} D{d} P{P}"
+        print(label, flush=True)
+        view = flat[offset:offset + q.numel()].view(q.shape)
+        view.copy_(q)
+        out = plan.run(view)
+        torch.cuda.synchronize()
+        _check(out, ref, label)
