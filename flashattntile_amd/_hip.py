@@ -49,6 +49,7 @@ ROWS_LANE = 2
 EXPORTED_SYMBOLS = (
     "fat_abi_version",
     "fat_last_error",
+    "fat_stream_capture_id",
     "fat_paged_decode_workspace_bytes",
     "fat_paged_decode_counters_bytes",
     "fat_paged_decode_balanced_workspace_bytes",
@@ -339,6 +340,8 @@ def _load() -> None:
             _ERROR = f"{path} has ABI version {version}, expected {ABI_VERSION}; rebuild it"
             return
         lib.fat_last_error.restype = ctypes.c_char_p
+        lib.fat_stream_capture_id.restype = _c_i64
+        lib.fat_stream_capture_id.argtypes = [_c_vp]
         lib.fat_paged_decode_workspace_bytes.restype = ctypes.c_size_t
         lib.fat_paged_decode_workspace_bytes.argtypes = [_c_i32, _c_i32, _c_i32, _c_i32]
         lib.fat_paged_decode_balanced_workspace_bytes.restype = ctypes.c_size_t
@@ -533,6 +536,11 @@ def current_stream_handle(device: torch.device) -> int:
     # torch's raw handle of the current stream, without a Stream object
     index = device.index
     return int(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index))
+
+
+def stream_capture_id(stream: int) -> int:
+    """Id of the capture that the stream (a handle) is part of, 0: none."""
+    return lib().fat_stream_capture_id(stream)
 
 
 def decode_workspace_bytes(batch: int, num_heads: int, head_dim: int, split_k: int) -> int:

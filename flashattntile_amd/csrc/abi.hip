@@ -33,4 +33,14 @@ int launch_status(const char* what) {
 
 extern "C" int fat_abi_version(void) { return FAT_ABI_VERSION; }
 
+extern "C" int64_t fat_stream_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();  // a launch on the stream reports it
+    return 0;
+  }
+  return status == hipStreamCaptureStatusNone ? 0 : (int64_t)id;
+}
+
 extern "C" const char* fat_last_error(void) { return g_last_error; }

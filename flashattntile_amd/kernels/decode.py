@@ -30,6 +30,8 @@ callers (benchmarks, CUDA-graph-style capture loops) that validated once.
 
 from __future__ import annotations
 
+import contextlib
+import threading
 import warnings
 
 import torch
@@ -538,17 +540,54 @@ def paged_decode_attention_multi(
     return _decode(q, cache, scale, cfg, prepared, sc)
 
 
+# Streams, other than the one a plan was made on, whose workspace it keeps;
+# captures that find cleared counters ready.
+_MAX_STREAMS = 64
+_CAPTURE_COUNTERS = 4
+
+
+def _on_stream(stream: int, device: torch.device):
+    """Make the stream with this handle torch's current one."""
+    if stream == _hip.current_stream_handle(device):
+        return contextlib.nullcontext()
+    return torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device) if stream
+                             else torch.cuda.default_stream(device))
+
+
+class _StreamState:
+    """What the runs of a :class:`DecodeLaunch` on one stream, or in one
+    capture of it, use: their argument block, workspace and merge counters
+    (both None where the launch has no partitions to merge)."""
+
+    __slots__ = ("args", "workspace", "counters")
+
+    def __init__(self, args, workspace, counters) -> None:
+        self.args = type(args).from_buffer_copy(args)
+        _hip.set_workspace(self.args, workspace)
+        self.args.merge_counters = None if counters is None else counters.data_ptr()
+        self.workspace, self.counters = workspace, counters
+
+
 class DecodeLaunch:
     """A decode launch prepared once and run every step (plan / run).
 
     Construction validates ``q`` and ``cache`` (one synchronisation, as
     :func:`paged_decode_attention` does, unless ``max_len`` and
     ``total_pages`` are given), resolves the launch (``config``, else the
-    tuned store, else the heuristic), allocates the split-K workspace and
-    fills the ``fat_decode_args`` block.  :meth:`run` then only writes the
+    tuned store, else the heuristic), allocates the workspace and fills the
+    ``fat_decode_args`` block.  :meth:`run` then only writes the
     query and output addresses into that block and enqueues
     ``fat_paged_decode``: no validation, synchronisation or allocation, about
-    the cost of one ctypes call.  The page table and seq_lens are read on the
+    the cost of one ctypes call.
+
+    Runs on different streams, captured runs among them, may overlap: each
+    stream but the one that was current at construction, and each capture,
+    gets a workspace and merge counters of its own at its first run (the plan
+    keeps those of the last 64 streams, and a capture's as long as it lives:
+    it has to outlive its graphs, as the cache has).  Runs on one stream share
+    theirs; no two threads may run a plan on one stream at a time.
+
+    The page table and seq_lens are read on the
     device at every run, so the serving engine updates them in place.  ``q``
     and ``out`` passed to :meth:`run` must have the dtype, shape and strides
     of the ``q`` given here (``out``: contiguous).  ``q`` is ``[B, H, D]`` or
@@ -596,18 +635,51 @@ class DecodeLaunch:
                                       cache.page_size, self.softmax_scale, cfg["split_k"], k_scale=k_scale,
                                       v_scale=v_scale, waves_per_group=cfg["num_warps"] or 0,
                                       pages_per_split=cfg["pages_per_split"], kernel=_KERNEL_CODES[cfg["kernel"]])
-        need = _plan_workspace_bytes(self._args, cfg)
-        self.workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
-        # Zeroed merge counters of this launch (each run leaves them zero):
-        # the decode kernel merges its partitions itself.  Runs of one
-        # DecodeLaunch share them, as they share the workspace.
-        self.counters = (torch.zeros(_hip.decode_counters_bytes(q.shape[0] * q_len, q.shape[-2]) // 4,
-                                     dtype=torch.int32, device=q.device) if need else None)
-        _hip.set_workspace(self._args, self.workspace)
-        self._args.merge_counters = None if self.counters is None else self.counters.data_ptr()
+        self._need = _plan_workspace_bytes(self._args, cfg)
+        self._num_counters = _hip.decode_counters_bytes(q.shape[0] * q_len, q.shape[-2]) // 4
         self._keep = (cache, k_scale, v_scale)  # the argument block points into these
         self._shape, self._dtype = tuple(q.shape), q.dtype
         self._device = q.device
+        self._lock = threading.Lock()
+        self._states: dict[tuple[int, int], _StreamState] = {}
+        self._spare_counters: list[torch.Tensor] = []
+        stream = _hip.current_stream_handle(q.device)
+        self._home = (stream, _hip.stream_capture_id(stream) if self._need else 0)
+        if self._need and not self._home[1]:
+            # For this stream, and for captures, which then need no fill of
+            # their own (a launch more in every replay).
+            self._spare_counters = list(self._zero_counters(1 + _CAPTURE_COUNTERS))
+        home = self._add_state(self._home)
+        self.workspace, self.counters = home.workspace, home.counters
+
+    def _zero_counters(self, sets: int) -> torch.Tensor:
+        return torch.zeros(sets, self._num_counters, dtype=torch.int32, device=self._device)
+
+    def _state(self, stream: int) -> _StreamState:
+        key = (stream, _hip.stream_capture_id(stream) if self._need else 0)
+        return self._states.get(key) or self._add_state(key)
+
+    def _add_state(self, key: tuple[int, int]) -> _StreamState:
+        stream, capture = key
+        with self._lock:
+            state = self._states.get(key)
+            if state is not None:
+                return state
+            workspace = counters = None
+            if self._need:
+                # Allocated and cleared on the stream that uses them: their
+                # memory goes to another use only behind its last run there.
+                with _on_stream(stream, self._device):
+                    workspace = torch.empty(self._need, dtype=torch.uint8, device=self._device)
+                    if self._spare_counters and (capture or key == self._home):
+                        counters = self._spare_counters.pop()
+                    else:
+                        counters = self._zero_counters(1)[0]
+            eager = [k for k in self._states if not k[1] and k != self._home]
+            if not capture and len(eager) >= _MAX_STREAMS:
+                del self._states[eager[0]]
+            state = self._states[key] = _StreamState(self._args, workspace, counters)
+            return state
 
     def run(self, q: torch.Tensor, out: torch.Tensor | None = None, stream: int | None = None) -> torch.Tensor:
         """Decode ``q`` into ``out`` (default: a new tensor) on ``stream``
@@ -618,8 +690,11 @@ class DecodeLaunch:
             out = torch.empty_like(q)
         elif tuple(out.shape) != self._shape or out.dtype != self._dtype or not out.is_contiguous():
             raise ValueError(f"DecodeLaunch.run: out must be a contiguous {self._dtype} tensor of shape {self._shape}")
-        a = self._args
+        if stream is None:
+            stream = _hip.current_stream_handle(self._device)
+        state = self._state(stream)
+        a = state.args
         a.q = q.data_ptr()
         a.out = out.data_ptr()
-        _hip.decode_with_args(a, _hip.current_stream_handle(self._device) if stream is None else stream)
+        _hip.decode_with_args(a, stream)
         return out

@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-/* 17: fat_decode_args.workspace_bytes.
+/* 17: fat_decode_args.workspace_bytes; fat_stream_capture_id.
  * 16: fat_prefill_paged_args.v_workspace, .total_k and fat_prefill_paged_v_bytes:
  *     chunks of long contexts on the wide kernel, K read through the pages.
  * 15: fat_decode_args.balanced; fat_check_begin / fat_check_wait (one launch and one host poll per
@@ -421,6 +421,10 @@ typedef struct fat_append_args {
   int32_t quant_dtype; /* FAT_DTYPE_I8 or FAT_DTYPE_FP8E4M3 (with a copy) */
   int32_t advance;     /* 1 = seq_lens += 1 (the reference's behaviour)   */
 } fat_append_args;
+
+/* Id of the capture that `stream` is part of (positive, another one for each
+ * capture of the process), 0 when it isn't capturing or can't be asked. */
+int64_t fat_stream_capture_id(void* stream);
 
 /* ABI version of the loaded library (FAT_ABI_VERSION at build time). */
 int fat_abi_version(void);
