@@ -410,7 +410,7 @@ class Check:
 
     def __init__(self, device: torch.device) -> None:
         with torch.cuda.device(device):
-            self._host = torch.zeros(CHECK_HOST_WORDS, dtype=torch.int64, pin_memory=True)
+            self._host = torch.zeros(CHECK_HOST_WORDS, dtype=torch.int64, device="cpu", pin_memory=True)
         self._device = device
         self._args = CheckArgs()
         self._args.host = self._host.data_ptr()

@@ -141,3 +141,47 @@ def test_validated_calls_are_refused_under_capture():
         graph.capture_end()
     torch.cuda.synchronize()
     assert torch.equal(prefill_attention(q, q, q, cu, cu, 8, 8), want)
+
+
+@pytest.mark.parametrize("default", ["cuda", "meta"])
+def test_validated_calls_under_a_default_device(default):
+    """The page-locked words of a thread's first check, whatever device the
+    program has tensors made on by default."""
+    from flashattntile_amd import append_tokens, paged_decode_attention, paged_prefill_attention, quantize_cache
+
+    print(f"check under default device {default}", flush=True)
+    q = torch.randn(2, 4, 64, device=DEV, dtype=torch.float16)
+    pages = torch.randn(4, 16, 2, 64, device=DEV, dtype=torch.float16)
+    table = _i32([[0, 1], [2, 3]]).to(DEV)
+    cu = _i32([0, 2]).to(DEV)
+    cu2 = _i32([0, 1, 2]).to(DEV)
+
+    def cache():
+        return PagedKVCache(pages.clone(), pages.clone(), table, _i32([20, 5]).to(DEV), 16)
+
+    def calls(c):
+        yield prefill_attention(q, q, q, cu, cu, 2, 2)
+        yield paged_decode_attention(q, c)
+        yield paged_prefill_attention(q, c, cu2, 1)
+        yield quantize_cache(c, "int8")[1].k
+        append_tokens(c, pages[:2, 0].contiguous(), pages[:2, 1].contiguous())
+        yield c.k_cache
+
+    want = [t.clone() for t in calls(cache())]
+    caches = [cache() for _ in want]  # one per call: an error of one doesn't end the others
+    got, errors = {}, []
+
+    def run(i):  # a thread's own check and default device
+        torch.set_default_device(default)
+        try:
+            got[i] = [t.clone() for t in calls(caches[i])][i]
+        except Exception as exc:
+            errors.append((i, exc))
+
+    for i in range(len(want)):
+        thread = threading.Thread(target=run, args=(i,))
+        thread.start()
+        thread.join(60)
+    torch.cuda.synchronize()
+    assert not errors, errors
+    assert all(torch.equal(got[i], want[i]) for i in range(len(want)))
