@@ -993,10 +993,14 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     if constexpr (LANE) {
       // Rows past t_end hold other tokens' data: their scores are masked,
       // and zero V rows keep p * v = 0 (the per-load form reads zeros there).
+      // So do zero scales: a first unit can look its rows up before t_end is
+      // known, in table columns that the sequence may not use, whose pages'
+      // scales can be anything.
       if (t_begin + ((u + 1) << UL) > t_end) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
           const bool in = t_begin + (u << UL) + i * RPL + r < t_end;
+          if constexpr (KV != KV_SAME && !BAL) cur.vsc[i] = in ? cur.vsc[i] : 0.f;
 #pragma unroll
           for (int n = 0; n < NC; ++n)
 #pragma unroll

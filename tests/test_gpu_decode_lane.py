@@ -100,3 +100,32 @@ def test_unaligned_queries_keep_the_generic_kernel():
     ref = ref_attention_paged(q.cpu().float(), k.cpu().float(), v.cpu().float(), pt.cpu(), sl.cpu(),
                               return_fp32=True)
     assert_parity(out, ref, label="lane unaligned q")
+
+
+@pytest.mark.parametrize("d,P", [(64, 1), (128, 3), (256, 16)])
+@pytest.mark.parametrize("qdtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mode", ["int8", "float8_e4m3fn"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_lane_scales_of_unused_columns(mode, qdtype, d, P, bad):
+    """Table columns past a sequence's pages name a page that no sequence
+    holds and whose scales are not finite."""
+    k, v, pt, sl = make_paged(LENS, 2, d, P, torch.float32, seed=P + 7, device="cpu", extra_pages=1)
+    qk, sk = quant_ref.quantize_pages(k, mode)
+    qv, sv = quant_ref.quantize_pages(v, mode)
+    held = torch.zeros(k.shape[0], dtype=torch.bool)
+    for b, n in enumerate(LENS):
+        held[pt[b, :-(-n // P)].long()] = True
+    spare = int((~held).nonzero()[0])
+    for b, n in enumerate(LENS):
+        pt[b, -(-n // P):] = spare
+    q = make_query(len(LENS), 8, d, qdtype, seed=P + 8, device=DEV)
+    ref = ref_attention_paged(q.cpu(), quant_ref.dequantize_pages(qk, sk, qdtype),
+                              quant_ref.dequantize_pages(qv, sv, qdtype), pt, sl, return_fp32=True)
+    sk[spare], sv[spare] = bad, bad
+    cache = PagedKVCache(qk.to(DEV), qv.to(DEV), pt.to(DEV), sl.to(DEV), P)
+    for cfg in [{**_config(split, pps, P), "num_warps": w} for split, pps in PARTS for w in (4, 8)] + [{"balanced": 3}]:
+        label = f"lane {mode} {qdtype} D{d} P{P} {cfg}, scales of {bad} past the end"
+        print(label, flush=True)
+        out = paged_decode_attention_fp8(q, cache, {"k": sk.to(DEV), "v": sv.to(DEV)}, config=cfg)
+        torch.cuda.synchronize()
+        assert_parity(out, ref, label=label)
