@@ -398,10 +398,10 @@ def _plan_workspace_bytes(a, cfg) -> int:
 def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     """Launch with the resolved partitions, from the prepared block if there
     is one."""
-    q = q.contiguous()
     if prepared is None:
-        prepared = _decode_block(q, cache, scale, scales)
+        prepared = _decode_block(q.contiguous(), cache, scale, scales)
     a, out, keep = prepared
+    q = keep[0]  # the copy that the block points at, where q wasn't contiguous
     need = _balance(a, cfg)
     if need:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)

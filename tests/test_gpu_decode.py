@@ -338,3 +338,42 @@ def test_decode_strided_page_table_and_seq_lens(layout):
     assert_parity(got, _ref32(q, cache), label=f"decode strided table {layout}")
     with pytest.raises(ValueError, match="contiguous"):
         DecodeLaunch(q, strided)
+
+
+@pytest.mark.parametrize("kind", ["same", "int8", "multi"])
+@pytest.mark.parametrize("split", [1, 3])
+def test_strided_query_is_copied_once(kind, split):
+    """A query view with gaps between its rows: one dense copy per call, and
+    the contiguous query's exact bits."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from flashattntile_amd import paged_decode_attention_fp8, paged_decode_attention_multi, quantize_cache
+
+    copies = []
+
+    class Count(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            if func.overloadpacket in (torch.ops.aten.clone, torch.ops.aten.copy_, torch.ops.aten._to_copy):
+                copies.append(func)
+            return func(*args, **(kwargs or {}))
+
+    _, cache = _case([700, 33, 4, 400], 8, 2, 128, 16, torch.float16, seed=43)
+    shape = (4, 3, 8, 128) if kind == "multi" else (4, 8, 128)
+    g = torch.Generator(device=DEV).manual_seed(44)
+    strided = torch.randn(*shape[:-1], 192, generator=g, device=DEV, dtype=torch.float16)[..., :128]
+    assert not strided.is_contiguous()
+    config = {"split_k": split}
+    if kind == "int8":
+        cache, scales = quantize_cache(cache, "int8")
+        call = lambda q: paged_decode_attention_fp8(q, cache, scales, config=config)
+    elif kind == "multi":
+        call = lambda q: paged_decode_attention_multi(q, cache, config=config)
+    else:
+        call = lambda q: paged_decode_attention(q, cache, config=config)
+    want = call(strided.contiguous())
+    call(strided)
+    with Count():
+        got = call(strided)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert len(copies) == 1, copies
