@@ -825,10 +825,12 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     }
   };
 
+  // Finite, so that a wave whose first units hold only scores of -inf gets
+  // p = 2^(-inf) = 0 for them, and not the NaN of -inf - -inf.
   float m_run[HPL], l_run[HPL];
 #pragma unroll
   for (int hh = 0; hh < HPL; ++hh) {
-    m_run[hh] = -INFINITY;
+    m_run[hh] = -__FLT_MAX__;
     l_run[hh] = 0.f;
   }
   float acc[HG][EPL];

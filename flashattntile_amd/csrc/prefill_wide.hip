@@ -206,7 +206,7 @@ void prefill_wide_kernel(const PrefillParams p) {
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[rb][db][r] = 0.f;
-  float m_run[2] = {-INFINITY, -INFINITY};
+  float m_run[2] = {-__FLT_MAX__, -__FLT_MAX__};  // finite: a first tile of scores of -inf gives p = 0, not NaN
   float l_run[2] = {0.f, 0.f};
   const int e_acc = VH ? p.v_head_scale[b * p.Hkv + kvh] : 0;  // bf16: O = acc * 2^e_acc
 

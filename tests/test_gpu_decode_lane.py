@@ -129,3 +129,35 @@ def test_lane_scales_of_unused_columns(mode, qdtype, d, P, bad):
         out = paged_decode_attention_fp8(q, cache, {"k": sk.to(DEV), "v": sv.to(DEV)}, config=cfg)
         torch.cuda.synchronize()
         assert_parity(out, ref, label=label)
+
+
+def _hide(q, k, pt, P, spans):
+    """Scores of -inf for the tokens of ``spans`` (per sequence): dim 0 of their
+    K is -inf, and that of every query is positive."""
+    q[..., 0] = q[..., 0].abs() + 0.5
+    for b, (lo, hi) in spans:
+        for t in range(lo, hi):
+            k[int(pt[b, t // P]), t % P, :, 0] = -float("inf")
+
+
+@pytest.mark.parametrize("P", [1, 3, 16])
+@pytest.mark.parametrize("dtype,d", [(torch.float16, 32), (torch.float16, 128), (torch.bfloat16, 64),
+                                     (torch.bfloat16, 256), (torch.float32, 64)])
+def test_units_of_minus_infinity(dtype, d, P):
+    """Whole units, waves and partitions whose scores are -inf beside others
+    that are not, as the generic kernel takes them (its 32-token tiles hold
+    finite scores first)."""
+    lens = [600, 130, 700]
+    k, v, pt, sl = make_paged(lens, 2, d, P, dtype, seed=d + P, device="cpu", poison=False)
+    q = make_query(len(lens), 8, d, dtype, seed=d, device="cpu")
+    _hide(q, k, pt, P, [(0, (64, 320)), (1, (32, 128)), (2, (256, 700))])
+    ref = ref_attention_paged(q.float(), k.float(), v.float(), pt, sl, return_fp32=True)
+    assert torch.isfinite(ref).all()
+    cache = PagedKVCache(k.to(DEV), v.to(DEV), pt.to(DEV), sl.to(DEV), P)
+    for cfg in ({"split_k": 1, "num_warps": 4}, {"split_k": 1, "num_warps": 8}, {"split_k": 3}, {"split_k": 20},
+                {"balanced": 4}, {"split_k": 1, "kernel": "generic"}):
+        label = f"-inf units D{d} {dtype} P{P} {cfg}"
+        print(label, flush=True)
+        out = paged_decode_attention(q.to(DEV), cache, config=cfg)
+        torch.cuda.synchronize()
+        _check(out, ref, label)

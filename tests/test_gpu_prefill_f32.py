@@ -95,3 +95,36 @@ def test_f32_prefill_no_further_from_64_bits_than_the_generic_kernel(d):
             errs[i] += (o[:, hh].double() - ref).square().sum().item() / ref.square().sum().item()
     print(f"matrix {errs[0] ** 0.5:.3e} valu {errs[1] ** 0.5:.3e}", flush=True)
     assert errs[0] ** 0.5 <= 1.2 * errs[1] ** 0.5
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_f32_prefill_infinite_scores(d, causal):
+    """Tiles whose scores are all -inf (the first, one wave's every tile), a
+    row that sees nothing else (zeros), and scores of +inf (NaN), beside the
+    generic kernel on the same inputs."""
+    print(f"f32 prefill infinite scores D{d} causal={causal}", flush=True)
+    lens = [300, 200]
+    q, k, v, cq, ck = _case(lens, lens, 4, 2, d, seed=d)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    k[0:32, :, 0] = -float("inf")  # the first tile of sequence 0
+    k[160:192, :, 0] = -float("inf")
+    for t in range(1, 6, 4):  # the tiles that one wave takes of sequence 1
+        k[300 + 32 * t:300 + min(32 * t + 32, 200), :, 0] = -float("inf")
+    args = (q, k, v, cq, ck)
+    out = prefill_attention(*args, max(lens), max(lens), causal=causal)
+    gen = prefill_attention(*args, max(lens), max(lens), causal=causal, config={"kernel": "generic"})
+    torch.cuda.synchronize()
+    if causal:  # rows 0 - 31 of sequence 0 see only hidden keys
+        assert (out[:32] == 0).all() and (gen[:32] == 0).all()
+    ref = ref_attention_varlen(q.cpu(), k.cpu(), v.cpu(), cq.cpu(), ck.cpu(), causal=causal)
+    for got in (out, gen):
+        seen = slice(32 if causal else 0, None)
+        rel = ((got.cpu() - ref).abs() / ref.abs().clamp_min(1.0))[seen].max().item()
+        assert torch.isfinite(got).all() and rel <= RTOL, rel
+    k[100, :, 0] = float("inf")
+    out = prefill_attention(*args, max(lens), max(lens), causal=causal)
+    gen = prefill_attention(*args, max(lens), max(lens), causal=causal, config={"kernel": "generic"})
+    torch.cuda.synchronize()
+    assert torch.equal(out.isnan(), gen.isnan()) and out[100:300].isnan().all() and not out[300:].isnan().any()
+    assert out[:100].isnan().any() != causal

@@ -86,3 +86,21 @@ def test_wide_paged_prefill_large_v_and_scales(scale):
                   label="large V, other elements")
     rel = ((out.float().cpu() - ref).abs() / ref.abs().clamp_min(1.0))[big].max().item()
     assert rel <= 2 * 2 ** -8 + 4e-3, rel  # two bf16 roundings
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_wide_paged_prefill_first_tile_of_minus_infinity(dtype, causal):
+    """A sequence whose first 32 keys, the wide kernel's first tile, all have
+    scores of -inf (the ping-pong kernel's first tile holds 64)."""
+    label = f"wide paged prefill -inf first tile {dtype} causal={causal}"
+    print(label, flush=True)
+    q, cache, cu, mq = _launch(SHORT, 32, 8, 16, dtype, seed=9)
+    q[..., 0] = q[..., 0].abs() + 0.5
+    for b in (0, 3):
+        cache.k_cache[cache.page_table[b, :2].long(), :, :, 0] = -float("inf")
+    out = paged_prefill_attention(q, cache, cu, mq, causal=causal)
+    pp = paged_prefill_attention(q, cache, cu, mq, causal=causal, config={"kernel": "pingpong"})
+    torch.cuda.synchronize()
+    assert_parity(out, _ref32(q, cache, cu, causal), label=label)
+    assert_parity(out, pp.float().cpu(), tol=4e-3, label=label + " vs ping-pong")
