@@ -206,7 +206,7 @@ void prefill_wide_kernel(const PrefillParams p) {
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[rb][db][r] = 0.f;
-  float m_run[2] = {-__FLT_MAX__, -__FLT_MAX__};  // finite: a first tile of scores of -inf gives p = 0, not NaN
+  float m_run[2] = {-INFINITY, -INFINITY};
   float l_run[2] = {0.f, 0.f};
   const int e_acc = VH ? p.v_head_scale[b * p.Hkv + kvh] : 0;  // bf16: O = acc * 2^e_acc
 
@@ -388,7 +388,7 @@ void prefill_wide_kernel(const PrefillParams p) {
       }
     return lsq[0] + lsq[1];
   };
-  auto exact_p = [&]() __attribute__((always_inline)) {
+  auto exact_p = [&](bool first) __attribute__((always_inline)) {
     float ls[2];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -397,6 +397,7 @@ void prefill_wide_kernel(const PrefillParams p) {
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[rb][r]);
       mx = xor32<OpMax>(mx);
       mx *= c;
+      if (PAGED && first) mx = fmaxf(mx, -__FLT_MAX__);  // finite: scores of -inf alone give p = 0, not NaN
       const bool grow = mx > m_run[rb] + kLazyPP;
       if (__any(grow)) {
         const float alpha = grow ? fast_exp2(m_run[rb] - mx) : 1.f;
@@ -415,7 +416,7 @@ void prefill_wide_kernel(const PrefillParams p) {
   auto softmax = [&](int t, int kbuf) __attribute__((always_inline)) {
     prep(t);
     if (t == 0) {
-      exact_p();
+      exact_p(true);
       return;
     }
     const float ls0 = compute_p(0);
@@ -423,7 +424,7 @@ void prefill_wide_kernel(const PrefillParams p) {
     if (__any(!(ls0 <= kLazyPPSum) || !(ls1 <= kLazyPPSum))) {  // rare; also catches inf / NaN
       qk(kbuf);
       prep(t);
-      exact_p();
+      exact_p(false);
       return;
     }
     l_run[0] += ls0;
