@@ -366,7 +366,11 @@ void prefill_wide_kernel(const PrefillParams p) {
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
         const int lim = CAUSAL ? min(kv_len - 1, max(row0 + 32 * rb + li, 0) + shift) : kv_len - 1;
-        const int rel = lim - n0 - 4 * g;
+        int rel = lim - n0 - 4 * g;
+        // Not causal, both blocks compare alike, and 16 masks kept for the
+        // second take 32 scalar registers: the paged bf16 form spilled (12
+        // bytes of scratch per lane).
+        if constexpr (!CAUSAL && PAGED && VH) __asm__ volatile("" : "+v"(rel));
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[rb][r] = ((r & 3) + 8 * (r >> 2)) <= rel ? s[rb][r] : -INFINITY;
       }
