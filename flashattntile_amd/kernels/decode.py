@@ -360,11 +360,12 @@ def _launch_block(a, q, split_k, workspace=None, waves_per_group=None, pages_per
     need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], split_k) if split_k > 1 else 0
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    a.workspace = None if workspace is None else workspace.data_ptr()
+    a.workspace_bytes = need  # held, as just checked
     # fat_paged_decode_counters_bytes: one int32 per (query row, head)
     if counters is not None and counters.numel() * counters.element_size() < 4 * rows * q.shape[-2]:
         raise ValueError("paged_decode_launch: counters smaller than decode_counters_bytes(rows, num_heads)")
     a.split_k = int(split_k)
-    _hip.set_workspace(a, workspace)
     a.waves_per_group = waves_per_group or 0
     a.pages_per_split = int(pages_per_split)
     a.kernel = _KERNEL_CODES[kernel]
@@ -405,7 +406,7 @@ def _decode(q, cache, scale, cfg, prepared, scales=None) -> torch.Tensor:
     need = _balance(a, cfg)
     if need:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-        _hip.set_workspace(a, workspace)
+        a.workspace, a.workspace_bytes = workspace.data_ptr(), need
         a.merge_counters = merge_counters(q, 2).data_ptr()
         _hip.decode_with_args(a, _hip.current_stream_handle(q.device))
         del keep
@@ -642,13 +643,15 @@ class DecodeLaunch:
         self._device = q.device
         self._lock = threading.Lock()
         self._states: dict[tuple[int, int], _StreamState] = {}
-        self._spare_counters: list[torch.Tensor] = []
+        self._cleared: torch.Tensor | None = None
+        self._cleared_sets = 0
         stream = _hip.current_stream_handle(q.device)
         self._home = (stream, _hip.stream_capture_id(stream) if self._need else 0)
         if self._need and not self._home[1]:
             # For this stream, and for captures, which then need no fill of
             # their own (a launch more in every replay).
-            self._spare_counters = list(self._zero_counters(1 + _CAPTURE_COUNTERS))
+            self._cleared_sets = 1 + _CAPTURE_COUNTERS
+            self._cleared = self._zero_counters(self._cleared_sets)
         home = self._add_state(self._home)
         self.workspace, self.counters = home.workspace, home.counters
 
@@ -671,13 +674,15 @@ class DecodeLaunch:
                 # memory goes to another use only behind its last run there.
                 with _on_stream(stream, self._device):
                     workspace = torch.empty(self._need, dtype=torch.uint8, device=self._device)
-                    if self._spare_counters and (capture or key == self._home):
-                        counters = self._spare_counters.pop()
+                    if self._cleared_sets and (capture or key == self._home):
+                        self._cleared_sets -= 1
+                        counters = self._cleared[self._cleared_sets]
                     else:
                         counters = self._zero_counters(1)[0]
-            eager = [k for k in self._states if not k[1] and k != self._home]
-            if not capture and len(eager) >= _MAX_STREAMS:
-                del self._states[eager[0]]
+            if not capture and len(self._states) > _MAX_STREAMS:
+                eager = [k for k in self._states if not k[1] and k != self._home]
+                if len(eager) >= _MAX_STREAMS:
+                    del self._states[eager[0]]
             state = self._states[key] = _StreamState(self._args, workspace, counters)
             return state
 
