@@ -1,5 +1,6 @@
-"""The fused paged-cache validation reductions (``fat_cache_stats``) against
-the torch reductions of the same quantities on the CPU copies: seq_lens
+"""The paged-cache validation's numbers, by the check kernel that the package
+runs and by ``fat_cache_stats`` of the C library, against the torch reductions
+of the same quantities on the CPU copies: seq_lens
 range, the page-table range over the columns the longest sequence uses
 (flashattn_tile/paging.py:123-129) and the page count, including batches
 above one workgroup's 1024 threads, empty and over-capacity sequences,
@@ -7,10 +8,12 @@ negative and out-of-pool ids, and a strided table."""
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
-from flashattntile_amd import PagedKVCache
+from flashattntile_amd import PagedKVCache, _hip
 from flashattntile_amd.paging import cache_stats
 
 pytestmark = pytest.mark.gpu
@@ -22,11 +25,25 @@ def _cache(lens, table, page_size, num_pages=64):
     return PagedKVCache(k, k, table, torch.tensor(lens, dtype=torch.int32), page_size)
 
 
+def _by_cache_stats(lens, table, page_size):
+    out = torch.full((5,), -99, dtype=torch.int64, device=DEV)
+    a = _hip.CacheStatsArgs()
+    a.seq_lens, a.page_table, a.out = lens.data_ptr(), table.data_ptr(), out.data_ptr()
+    a.batch, a.max_pages, a.page_size, a.page_table_stride = *table.shape, page_size, table.stride(0)
+    stream = ctypes.c_void_p(_hip.current_stream_handle(lens.device))
+    assert _hip.lib().fat_cache_stats(ctypes.byref(a), stream) == 0, _hip.lib().fat_last_error()
+    stats = out.tolist()
+    if stats[2] == torch.iinfo(torch.int32).max:  # no column in use
+        stats[2], stats[3] = 0, -1
+    return tuple(stats)
+
+
 def _both(lens, table, page_size):
     cpu = _cache(lens, table, page_size)
     want = cache_stats(cpu, with_total_pages=True)
     dev = PagedKVCache(cpu.k_cache.to(DEV), cpu.v_cache.to(DEV), table.to(DEV), cpu.seq_lens.to(DEV), page_size)
     got = cache_stats(dev, with_total_pages=True)
+    assert _by_cache_stats(dev.seq_lens, dev.page_table, page_size) == got
     return got, want
 
 
