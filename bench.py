@@ -41,7 +41,7 @@ from flashattntile_amd.env import MI355X, peak_hbm_gbs, peak_mfma_tflops  # noqa
 
 HBM_PEAK_GBS = peak_hbm_gbs()
 MFMA_PEAK_TFLOPS = peak_mfma_tflops("fp16")  # dense fp16 / bf16
-VALU_FP32_PEAK_TFLOPS = MI355X["vector_fp32_tflops"]  # the generic fp32 prefill kernel's bound
+VALU_FP32_PEAK_TFLOPS = MI355X["vector_fp32_tflops"]  # fp32: vector and matrix rate alike
 MALL_BYTES = 256 << 20
 FLUSH_BYTES = 512 << 20
 
@@ -235,8 +235,10 @@ def _time_cpu(fn, budget_s, max_reps=21):
 # Headline legs
 # ---------------------------------------------------------------------------
 def _product_launch(q, pools, table, lens, page, max_len, total_pages, q_len=1):
-    """What the decode wrappers launch for this shape (tuned store, else the
-    heuristic): (split_k, pages_per_split, waves or 0, kernel code, source)."""
+    """The partitions that the decode wrappers launch for this shape (tuned
+    store, else the heuristic): (split_k, pages_per_split, waves or 0, kernel
+    code, source).  Rows here are uniform, short or in the store, so none runs
+    as a balanced launch (checked)."""
     from flashattntile_amd import PagedKVCache, _hip
     from flashattntile_amd.autotune import best_config, decode_signature
     from flashattntile_amd.kernels.decode import resolve_decode_config
@@ -244,6 +246,8 @@ def _product_launch(q, pools, table, lens, page, max_len, total_pages, q_len=1):
     k, v = pools[0][0], pools[0][1]
     cache = PagedKVCache(k, v, table, lens, page)
     cfg = resolve_decode_config(q, cache, max_len, total_pages, q_len=q_len)
+    if cfg["balanced"]:
+        raise SystemExit("bench.py: the wrappers run this batch balanced, and this row would time its partitions")
     sig = decode_signature(q.shape[0], q.shape[-2], k.shape[2], q.shape[-1], page, max_len, total_pages, k.dtype,
                            q_len)
     source = "tuned store" if best_config("decode", sig) else "heuristic"
@@ -964,9 +968,9 @@ def all_configs(args, device):
         for L in (512, 1024, 2048, 4096, 8192):
             emit(_prefill_row(f"prefill {dn} causal L{L}", [L], dt, device, args))
         emit(_prefill_row(f"prefill {dn} causal mixed8 {sum(mixed)} tok", mixed, dt, device, args))
-    # fp32 prefill: the generic VALU kernel (its bound is the 157.3 TFLOP/s fp32 vector peak)
+    # fp32 prefill: the fp32 matrix kernel (its bound is the 157.3 TFLOP/s of fp32 MFMAs)
     for L in (1024, 4096):
-        emit(_prefill_row(f"prefill fp32 causal L{L} (generic)", [L], torch.float32, device, args))
+        emit(_prefill_row(f"prefill fp32 causal L{L}", [L], torch.float32, device, args))
     # quantised decode B128 ctx16384
     for mode, mn in (("int8", "int8"), ("float8_e4m3fn", "fp8")):
         emit(_decode_row(f"decode {mn} B128 ctx16384", [16384] * 128, 32, 8, 128, 16, device, args, flush,
@@ -982,12 +986,12 @@ def all_configs(args, device):
     emit(_decode_row("decode fp16 D64 B32 ctx4096", [4096] * 32, 32, 8, 64, 16, device, args, flush))
     for page in (32, 64):
         emit(_decode_row(f"decode fp16 P{page} B32 ctx4096", [4096] * 32, 32, 8, 128, page, device, args, flush))
-    # the generic decode kernel (LDS-tiled, any page size): fp32, and pages of 1 and 5 rows
+    # the VALU decode's per-lane form: fp32, and pages of 1 and 5 rows
     for dt, dn in ((torch.float32, "fp32"), (torch.float16, "fp16")):
         for page in (1, 5):
-            emit(_decode_row(f"decode {dn} generic P{page} B32 ctx4096", [4096] * 32, 32, 8, 128, page, device,
+            emit(_decode_row(f"decode {dn} P{page} B32 ctx4096", [4096] * 32, 32, 8, 128, page, device,
                              args, flush, dtype=dt))
-    emit(_decode_row("decode fp32 generic P16 B32 ctx4096", [4096] * 32, 32, 8, 128, 16, device, args, flush,
+    emit(_decode_row("decode fp32 P16 B32 ctx4096", [4096] * 32, 32, 8, 128, 16, device, args, flush,
                      dtype=torch.float32))
     # Multi-token (speculative) decode: T query tokens per sequence
     for T in (2, 4, 8):

@@ -243,8 +243,10 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
       library chooses for longer whole sequences.
 
     Measured with 120 drawn batches against every split_k of 1-32 and both
-    numbers of waves; :func:`decode_partition`, which this replaces for the
-    library's own choice, was 1.1-2 times slower than the best of them.
+    numbers of waves; :func:`decode_partition`, which this replaces where the
+    wrappers choose, was 1.1-2 times slower than the best of them.  The tuned
+    store's entries, chosen against that rule's launch, go before this one,
+    and the native entry, which doesn't know the lengths, still takes it.
     """
     items = max(1, int(items))
     split = 1

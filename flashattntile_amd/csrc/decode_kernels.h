@@ -649,7 +649,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
   const int c = lane % LPR;
 
   // One partition (or, BAL, one segment: tokens [seg_begin, seg_end)) of
-  // sequence b and head group y.
+  // sequence b and head group y: the kernel's body, to "// segment".
   auto segment = [&](const DecodeParams& p, const int b, const int y, const int split, const int S, const int seg_begin, const int seg_end,
                      const int slot, const int item, const int w_first, const int n_parts)
       __attribute__((always_inline)) {
@@ -659,8 +659,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
   const int nvalid = min(HG, p.group - sub * HG);
 
   // Page ids of this wave's first unit, read together with seq_len when
-  // `early` (first_page_ids); rows of that unit past the sequence's end read
-  // the table again (fetch).
+  // `early` (first_page_ids).
   constexpr int UL = Gm::kUnitLog2;
   const int32_t* ptrow = p.pt + (int64_t)b * p.pt_sb;
   const bool early = !BAL && (split == 0 || p.pps_fixed > 0);
@@ -1089,7 +1088,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
       o = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
     });
   }
-  };
+  };  // segment
 
   if constexpr (BAL) {
     constexpr int WB = Gm::kUnitLog2 + (NW == 8 ? 3 : 2);  // a block: one unit per wave
@@ -1151,7 +1150,7 @@ void paged_decode_mfma_kernel(const DecodeParams p) {
   const int li = lane & 31;  // key row (A operand) / (head, token) column (B, S^T)
   const int g = lane >> 5;   // k-group: head dims 16ks + 8g .. +7 of k-step ks
 
-  // One partition, or segment (see paged_decode_kernel).
+  // One partition, or segment (see paged_decode_kernel), to "// segment".
   auto segment = [&](const DecodeParams& p, const int b, const int y, const int split, const int S, const int seg_begin, const int seg_end,
                      const int slot, const int item, const int w_first, const int n_parts)
       __attribute__((always_inline)) {
@@ -1482,7 +1481,7 @@ void paged_decode_mfma_kernel(const DecodeParams p) {
       o = (int64_t)b * p.o_sb + (int64_t)tt * p.o_st + (int64_t)h * p.o_sh;
     });
   }
-  };
+  };  // segment
 
   if constexpr (BAL) {
     constexpr int WB = 5 + (NW == 8 ? 3 : 2);  // a block: 32 keys per wave

@@ -1,12 +1,16 @@
-// validate.hip -- the device half of the paged-cache validation: one launch
-// reduces seq_lens and the used page-table entries to the five numbers the
-// host checks (flashattn_tile/paging.py:84-130 validate_cache, as called by
-// flashattn_tile/kernels/decode.py:503-522), instead of a dozen framework
-// reductions.  The host copies the five numbers back once.
+// validate.hip -- the device half of the validation: one launch reduces the
+// lengths, offsets and used page-table entries that a call is to check
+// (flashattn_tile/paging.py:84-130 validate_cache, as called by
+// flashattn_tile/kernels/decode.py:503-522, and kernels/prefill.py:194-233)
+// to a few numbers, instead of a dozen framework reductions.
 //
-// fat_check_begin / fat_check_wait do that for every validated call without
-// the copy and the synchronisation: the kernel writes its numbers into
-// page-locked host memory and the host polls them.
+// fat_check_begin / fat_check_wait: what the Python package runs.  The kernel
+// writes its numbers into page-locked host memory and the host polls them, so
+// a validated call neither copies nor synchronises.
+//
+// fat_cache_stats: the same numbers of a paged cache in device memory, for
+// callers of the C library that have no page-locked words or copy them with
+// other results.
 #include <limits.h>
 
 #include <algorithm>

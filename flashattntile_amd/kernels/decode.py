@@ -20,9 +20,12 @@ Differences, all deliberate:
 * ``config=None`` takes the launch stored for this shape in the gfx950
   tuned-config store (:func:`flashattntile_amd.autotune.best_config`, keyed by
   :func:`~flashattntile_amd.autotune.decode_signature`) and otherwise the
-  MI355X partition heuristic (:func:`~flashattntile_amd.autotune.decode_partition`);
-  an explicit ``split_k`` is honoured exactly;
-* validation costs one device->host synchronisation instead of ~6.
+  MI355X heuristics: balanced runs
+  (:func:`~flashattntile_amd.autotune.decode_balanced`) or partitions
+  (:func:`~flashattntile_amd.autotune.decode_split`); an explicit ``split_k``
+  is honoured exactly;
+* validation costs one check launch that the host polls while it prepares the
+  decode, instead of ~6 device->host synchronisations.
 
 :func:`paged_decode_launch` is the sync-free entry below the validation, for
 callers (benchmarks, CUDA-graph-style capture loops) that validated once.

@@ -16,9 +16,12 @@ on the host before anything is enqueued.  What the binding accepts, this does:
   of the Python wrappers' error.
 
 The library picks the kernel: the VALU/MFMA decode where it takes the shape,
-the generic decode (fp32, pages below the fast kernels' floor or not a power
-of two) otherwise.  The launch needs no device synchronisation: the split-K
-partition comes from the page table's width, not from the lengths.
+the VALU kernel's per-lane form (fp32, pages below the fast kernels' floor or
+not a power of two) otherwise.  The launch needs no device synchronisation:
+the split-K partition comes from the page table's width, not from the lengths,
+so it is that of :func:`~flashattntile_amd.autotune.decode_partition` and not
+of the rule that knows them
+(:func:`~flashattntile_amd.autotune.decode_split`).
 """
 
 from __future__ import annotations

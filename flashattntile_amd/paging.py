@@ -241,7 +241,8 @@ def append_tokens(cache: PagedKVCache, new_k: torch.Tensor, new_v: torch.Tensor,
     (the reference has no incremental form; it requantises the whole cache).
 
     On a ROCm cache the write (and the requantisation) is the HIP kernel
-    ``fat_append_kv``; the bounds checks cost one device synchronisation.
+    ``fat_append_kv``; the bounds checks cost one check launch that the host
+    polls.
     ``validate=False`` skips them (ROCm only): an entry whose position or page
     id is out of range is then skipped on the device and its length kept.
     """
@@ -289,8 +290,9 @@ def append_tokens(cache: PagedKVCache, new_k: torch.Tensor, new_v: torch.Tensor,
 
 
 def _append_hip(cache: PagedKVCache, new_k: torch.Tensor, new_v: torch.Tensor, mirror, validate: bool) -> None:
-    """ROCm path of :func:`append_tokens`: bounds checks in one copy, then
-    ``fat_append_kv`` on the current stream."""
+    """ROCm path of :func:`append_tokens`: bounds checks by one launch that
+    the host polls (``fat_check_begin``), then ``fat_append_kv`` on the current
+    stream."""
     from . import _hip
 
     dev = cache.k_cache.device
