@@ -212,13 +212,15 @@ def decode_partition(batch: int, num_heads: int, num_kv_heads: int, max_pages: i
 
 
 def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: int, mfma: bool = False,
-                 shared: bool = False, num_cus: int = MI355X_CUS) -> tuple[int, int | None]:
+                 shared: bool = False, num_cus: int = MI355X_CUS, rows: int = 4,
+                 waves: int | None = None) -> tuple[int, int | None]:
     """``(split_k, waves)`` of a decode launch with ``split_k`` equal
     partitions of every sequence: ``items`` (sequence, head group) pairs, each
     one workgroup when it isn't split, over ``mean_len`` tokens on average and
     ``max_len`` at most, ``item_token_bytes`` of K and V per token and head
-    group, on the MFMA kernel or a VALU one; ``shared``: several head groups
-    read the same lines of K and V.  Waves None: the library's choice.
+    group, ``rows`` (head, token) rows per workgroup, on the MFMA kernel or a
+    VALU one; ``shared``: several head groups read the same lines of K and V;
+    ``waves``: what the caller asks for.  Waves None: the library's choice.
 
     * As many partitions as fill the CUs once, no shorter than 128 tokens and
       none below 256: a small launch is latency along its longest partition
@@ -237,6 +239,19 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
       512 tokens and more, and so have those whose head groups share lines: 40
       sequences of 4500 tokens, 8 head groups, int8 at head_dim 64, 85.2 ->
       65.8 us, 54 of 1950 with 8 head groups per KV head 74 -> 55.
+    * Batches whose longest sequence is four times the mean or more have a
+      rule of their own.  To twelve times, lengths spread over decades: many
+      long sequences share their CUs and run on when the others are done, so a
+      CU's share of the tokens is 2.5 partitions (3 on the VALU kernels, 5 of
+      a single row; half as many of eight waves).  Beyond, a few long contexts
+      among short ones: 1.2 shares, as above.  No shorter than 2000 tokens, in
+      a grid of at most 20 workgroups per CU (24 on the VALU kernels, 32
+      around one very long sequence).  Workgroups of more than 16 rows, fewer
+      and slower, take partitions of 2048 tokens.  Against the rule above
+      (measured on lengths within a factor of 30): 128 log-uniform lengths in
+      [16, 16384], 64/8 heads 368 -> 291 us, int8 at head_dim 64 182 -> 138,
+      four tokens each 372 -> 316; one of 100000 and 63 of 200, 32/1 heads 166
+      -> 67; 2 of 65536 and 30 of 512 88 -> 48; 100 in [100, 10000] 57 -> 47.
     * Eight waves where a CU has one workgroup, but four on the VALU kernels
       for whole sequences below 1024 tokens (240 items of 609 tokens 17.3 ->
       16.8 us, 33 x 8 of 68 11.4 -> 7.8) and in larger grids, except that the
@@ -255,6 +270,17 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
         if 16 * items <= num_cus // 2 and max_len >= 4096:
             cap = 64 if max_len >= 65536 else 32
         split = max(1, min(num_cus // items, -(-max_len // 128), cap))
+    if max_len >= 4 * mean_len and max_len * item_token_bytes > 10 * 40e3:
+        if rows > 16:
+            split = max(split, min(-(-max_len // 2048), 32))
+            return split, 8 if items * split <= 3 * num_cus else 4
+        need = max_len * num_cus / (items * max(mean_len, 1.0))  # partitions of one CU's share each
+        grid = 32 * num_cus if need > 16 else (20 if mfma else 24) * num_cus
+        spread = max_len < 12 * mean_len
+        per_share = (2.5 if mfma else 5.0 if rows == 1 else 3.0) / (2 if waves == 8 else 1)
+        want = 1 if mfma and need < 1 else math.ceil(per_share * need if spread else need / 1.2)
+        split = max(split, min(want, -(-max_len // 2000), grid // items, 24))
+        return split, 8 if items * split <= num_cus else 4
     if max_len * item_token_bytes > 10 * 40e3:  # 40 GB/s per CU: bytes per us
         if max_len >= 1.25 * mean_len and items * mean_len * item_token_bytes > 15 * 6.2e6:
             need = max_len * num_cus / (1.2 * items * max(mean_len, 1.0))
@@ -270,17 +296,34 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
     return split, None if not mfma and split == 1 and max_len >= 1024 else 4
 
 
-def decode_balanced(max_len: int, mean_len: float, kv_bytes: int, rows: int) -> bool:
+def decode_balanced(max_len: int, mean_len: float, kv_bytes: int, rows: int, items: int = 1,
+                    item_token_bytes: int = 512, mfma: bool = False) -> bool:
     """Whether a decode launch of the library's own choice cuts the batch into
     equal runs (fat_decode_args.balanced) instead of :func:`decode_split`'s
     partitions, where its kernel has that form: ragged batches whose K/V
     (``kv_bytes``) take the memory 25 us or more, with at most 16 (head,
     token) ``rows`` per workgroup.  64 sequences of 500-16000 tokens on an fp8
-    cache 151 -> 130.5 us, 64 log-uniform in [16, 65536] in fp16 403 -> 351,
-    40 of 100-10000 at head_dim 64 49.8 -> 46.5; level at 20 of 300-5000
-    (126 MB), and behind on uniform batches, which partitions divide as well
-    without finding their place in the batch first.
+    cache 151 -> 130.5 us, one of 100000 and 63 of 200 in fp16 109 -> 93; level
+    at 20 of 300-5000 (126 MB) and, in fp16, at 64 log-uniform in [16, 65536]
+    (338 us; 334 in partitions of four waves, 312 of eight), and behind on
+    uniform batches, which partitions divide as well without finding their
+    place in the batch first.
+
+    Not where lengths spread over decades (the longest 4 to 12 times the mean)
+    and many items are short: an item costs a run more than its tokens do, so
+    runs of equal tokens aren't equal.  That is 512 ``items`` (sequence, head
+    group) or more of less than 750 KB on average, 1536 on the MFMA kernel (256
+    log-uniform in [16, 8192]: fp8 221 us balanced, 184 whole; 512 in [16,
+    4096] 361 and 327; 96 in [16, 6000] 93 and 89; but fp8 100 in [100, 10000]
+    95 and 106), and any number on the VALU kernels at 256 bytes per token and
+    less (head_dim 64: 256 as above 208 and 161, 64 in [64, 16384] 87 and 79, 32
+    in [16, 65536] 90 and 86).  A few long sequences among short ones stay
+    balanced (4 of 30000 and 124 of 1000: 171 and 188).
     """
+    if 4 * mean_len <= max_len < 12 * mean_len and (
+            (items >= (1536 if mfma else 512) and kv_bytes < 750e3 * items) or
+            (not mfma and item_token_bytes <= 256)):
+        return False
     return max_len >= 1.5 * mean_len and kv_bytes >= 150e6 and rows <= 16
 
 

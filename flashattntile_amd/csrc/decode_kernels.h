@@ -380,8 +380,10 @@ __device__ __forceinline__ void merge_in_launch(const DecodeParams& p, int S, in
 // 512 workgroups of four waves (768-2048: level to 20 % slower) against the
 // best partitions: 64 sequences of 500-16000 tokens, 32/8 heads, head_dim 128,
 // on an fp8 cache 151 -> 130.5 us (534 MB, 4.1 TB/s), on a bf16 one 228 ->
-// 201, 64 log-uniform in [16, 65536] in fp16 403 -> 351, 32 of 500-4000 with
-// pages of one token 54.5 -> 49.5.
+// 201, 32 of 500-4000 with pages of one token 54.5 -> 49.5, one of 100000 and
+// 63 of 200 in fp16 109 -> 93.  A run counts an item's tokens and not what an
+// item costs besides, so it loses where a batch holds many very short ones
+// (256 log-uniform in [16, 8192], head_dim 64, 161 -> 208).
 // ---------------------------------------------------------------------------
 
 // s_cum[b] = blocks of a head group's items over the sequences before b, for

@@ -163,7 +163,7 @@ def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: i
         if resolved["balanced"] is None and resolved["pages_per_split"] is None and waves in (None, 4) \
                 and balances:
             resolved["balanced"] = int(decode_balanced(max_len, mean_len, token_bytes * hkv * total_pages * page,
-                                                       rows))
+                                                       rows, items, token_bytes, mfma))
         if resolved["balanced"] or resolved["pages_per_split"] is not None:
             # what a kernel without the balanced form falls back to
             split, chunk = decode_partition(batch, heads, hkv, max_pages, total_pages,
@@ -177,7 +177,8 @@ def _merge_config(config: dict, q: torch.Tensor, cache: PagedKVCache, max_len: i
             if resolved["num_warps"] is None and is_ragged(batch, max_pages, total_pages):
                 resolved["num_warps"] = 4
         else:
-            resolved["split_k"], chosen = decode_split(items, max_len, mean_len, token_bytes, mfma, shared)
+            resolved["split_k"], chosen = decode_split(items, max_len, mean_len, token_bytes, mfma, shared,
+                                                       rows=rows, waves=waves)
             resolved["pages_per_split"] = 0
             if resolved["num_warps"] is None:
                 resolved["num_warps"] = chosen
