@@ -320,11 +320,11 @@ def decode_balanced(max_len: int, mean_len: float, kv_bytes: int, rows: int, ite
     in [16, 65536] 90 and 86).  A few long sequences among short ones stay
     balanced (4 of 30000 and 124 of 1000: 171 and 188).
     """
-    if 4 * mean_len <= max_len < 12 * mean_len and (
-            (items >= (1536 if mfma else 512) and kv_bytes < 750e3 * items) or
-            (not mfma and item_token_bytes <= 256)):
+    if max_len < 1.5 * mean_len or kv_bytes < 150e6 or rows > 16:
         return False
-    return max_len >= 1.5 * mean_len and kv_bytes >= 150e6 and rows <= 16
+    if not 4 * mean_len <= max_len < 12 * mean_len:
+        return True
+    return (items < (1536 if mfma else 512) or kv_bytes >= 750e3 * items) and (mfma or item_token_bytes > 256)
 
 
 def is_ragged(batch: int, max_pages: int, total_pages: int) -> bool:

@@ -361,7 +361,8 @@ def _launch_block(a, q, split_k, workspace=None, waves_per_group=None, pages_per
                   counters=None) -> None:
     """Enqueue the block of :func:`_decode_block` with these partitions."""
     rows = q.shape[0] * (q.shape[1] if q.dim() == 4 else 1)
-    need = _hip.decode_workspace_bytes(rows, q.shape[-2], q.shape[-1], split_k) if split_k > 1 else 0
+    # fat_paged_decode_workspace_bytes: (acc, m, l) per (query row, head, partition)
+    need = 4 * rows * q.shape[-2] * split_k * (q.shape[-1] + 2) if split_k > 1 else 0
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     a.workspace = None if workspace is None else workspace.data_ptr()

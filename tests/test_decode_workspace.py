@@ -84,3 +84,21 @@ def test_stated_workspace_is_not_exceeded():
     a.workspace_bytes = -1
     assert _hip.lib().fat_paged_decode(ctypes.byref(a), None) == 1
     assert "workspace_bytes" in _hip.lib().fat_last_error().decode()
+
+
+@pytest.mark.parametrize("split", [1, 2, 7, 64])
+def test_launch_sizes_its_partitions_as_the_library_does(split, monkeypatch):
+    from flashattntile_amd.kernels import decode as dec
+
+    seen = []
+    monkeypatch.setattr(_hip, "decode_with_args", lambda a, stream: seen.append((a.workspace, a.workspace_bytes)))
+    monkeypatch.setattr(_hip, "current_stream_handle", lambda device: 0)
+    for shape in ((3, 8, 128), (2, 5, 4, 64)):
+        q = torch.empty(*shape)
+        rows = shape[0] * (shape[1] if len(shape) == 4 else 1)
+        need = _hip.decode_workspace_bytes(rows, shape[-2], shape[-1], split)
+        dec._launch_block(_hip.DecodeArgs(), q, split)
+        held = torch.empty(max(1, need), dtype=torch.uint8)
+        dec._launch_block(_hip.DecodeArgs(), q, split, workspace=held)
+        assert [b for _, b in seen] == [need, need] and (split == 1 or seen[1][0] == held.data_ptr())
+        seen.clear()
