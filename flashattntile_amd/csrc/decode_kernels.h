@@ -781,12 +781,17 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_kernel(const DecodeParam
     for (int i = 0; i < NI; ++i) {
       const int rs = base + i * RPL;
       const int nrow = min(t_end - rs, RPL);  // rows of this load in the partition
-      // The table is read without a branch so that a unit's page-id loads
-      // issue together.  A load wholly past t_end reads no rows (range 0),
-      // and the page of a row before t_end: the scales of a column that the
-      // sequence doesn't use can be anything, and 0 * NaN would reach acc.
-      int phys = first && early ? (nrow > 0 ? first_pid[i] : first_pid[0])
-                                : uniform_load(ptrow, min(rs, t_end - 1) >> p.log2P);
+      // The table is read without a branch (at most its last entry) so that
+      // a unit's page-id loads issue together; a load wholly past t_end reads
+      // nothing (range 0).  8-bit caches: it names the page of a row before
+      // t_end, since the scales of a column that the sequence doesn't use can
+      // be anything, and 0 * NaN would reach acc.
+      int phys;
+      if constexpr (KV == KV_SAME)
+        phys = first && early ? first_pid[i] : uniform_load(ptrow, min(rs >> p.log2P, p.max_pages - 1));
+      else
+        phys = first && early ? (nrow > 0 ? first_pid[i] : first_pid[0])
+                              : uniform_load(ptrow, min(rs, t_end - 1) >> p.log2P);
       phys = __builtin_amdgcn_readfirstlane(min(max(phys, 0), p.num_pages - 1));
       const uint32_t slot0 = (uint32_t)(rs & (p.P - 1));
       // range: the load's rows inside the partition, each up to its head slice's end
@@ -1225,10 +1230,15 @@ void paged_decode_mfma_kernel(const DecodeParams p) {
     for (int i = 0; i < NLD; ++i) {
       const int rs = kb + i * RPL;
       const int nrow = min(t_end - rs, RPL);  // rows of this load in the partition
-      // read without a branch; a load wholly past t_end reads no rows (range
-      // 0) and the page of one before it (see paged_decode_kernel)
-      int phys = first && early ? (nrow > 0 ? first_pid[i] : first_pid[0])
-                                : uniform_load(ptrow, min(rs, t_end - 1) >> p.log2P);
+      // read without a branch (at most the table's last entry); a load wholly
+      // past t_end reads nothing (range 0), 8-bit caches the page of a row
+      // before it (see paged_decode_kernel)
+      int phys;
+      if constexpr (KV == KV_SAME)
+        phys = first && early ? first_pid[i] : uniform_load(ptrow, min(rs >> p.log2P, p.max_pages - 1));
+      else
+        phys = first && early ? (nrow > 0 ? first_pid[i] : first_pid[0])
+                              : uniform_load(ptrow, min(rs, t_end - 1) >> p.log2P);
       phys = __builtin_amdgcn_readfirstlane(min(max(phys, 0), p.num_pages - 1));
       const uint32_t slot0 = (uint32_t)(rs & (p.P - 1));
       const int nk = nrow > 0 ? (int)((uint32_t)(nrow - 1) * krow + EB * D) : 0;
