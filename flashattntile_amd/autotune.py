@@ -243,11 +243,13 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
       rule of their own.  To twelve times, lengths spread over decades: many
       long sequences share their CUs and run on when the others are done, so a
       CU's share of the tokens is 2.5 partitions (3 on the VALU kernels, 5 of
-      a single row; half as many of eight waves).  Beyond, a few long contexts
-      among short ones: 1.2 shares, as above.  No shorter than 2000 tokens, in
-      a grid of at most 20 workgroups per CU (24 on the VALU kernels, 32
-      around one very long sequence).  Workgroups of more than 16 rows, fewer
-      and slower, take partitions of 2048 tokens.  Against the rule above
+      a single row, 1.25 of more than 16, whose partials are large; half as
+      many of eight waves).  Beyond, a few long contexts among short ones: 1.2
+      shares, as above.  No shorter than 2000 tokens, in a grid of at most 20
+      workgroups per CU (24 on the VALU kernels, 32 around one very long
+      sequence).  Where fewer sequences than CUs have more than 16 rows (32/1
+      heads), each a long chain, partitions of 2048 tokens, to 8 per CU.
+      Against the rule above
       (measured on lengths within a factor of 30): 128 log-uniform lengths in
       [16, 16384], 64/8 heads 368 -> 291 us, int8 at head_dim 64 182 -> 138,
       four tokens each 372 -> 316; one of 100000 and 63 of 200, 32/1 heads 166
@@ -271,14 +273,15 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
             cap = 64 if max_len >= 65536 else 32
         split = max(1, min(num_cus // items, -(-max_len // 128), cap))
     if max_len >= 4 * mean_len and max_len * item_token_bytes > 10 * 40e3:
-        if rows > 16:
-            split = max(split, min(-(-max_len // 2048), 32))
+        if rows > 16 and items < num_cus:
+            split = max(split, min(int(max_len / 2048 + 0.5), 32, 8 * num_cus // items))
             return split, 8 if items * split <= 3 * num_cus else 4
         need = max_len * num_cus / (items * max(mean_len, 1.0))  # partitions of one CU's share each
-        grid = 32 * num_cus if need > 16 else (20 if mfma else 24) * num_cus
+        grid = 32 * num_cus if need > 16 and rows <= 16 else (20 if mfma else 24) * num_cus
         spread = max_len < 12 * mean_len
-        per_share = (2.5 if mfma else 5.0 if rows == 1 else 3.0) / (2 if waves == 8 else 1)
-        want = 1 if mfma and need < 1 else math.ceil(per_share * need if spread else need / 1.2)
+        per_share = (1.25 if rows > 16 else 2.5 if mfma else 5.0 if rows == 1 else 3.0) / (2 if waves == 8 else 1)
+        whole = mfma and need < (1.4 if rows > 16 else 1)
+        want = 1 if whole else math.ceil(per_share * need if spread else need / 1.2)
         split = max(split, min(want, -(-max_len // 2000), grid // items, 24))
         return split, 8 if items * split <= num_cus else 4
     if max_len * item_token_bytes > 10 * 40e3:  # 40 GB/s per CU: bytes per us

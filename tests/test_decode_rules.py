@@ -60,6 +60,8 @@ def test_decode_split_of_very_ragged_batches():
     assert decode_split(1024, 16000, 16000 / 6, 512, False)[0] > decode_split(1024, 16000, 16000 / 2, 512, False)[0]
     # one long sequence among short ones, 32 rows per workgroup
     assert decode_split(64, 100000, 1759, 512, True, rows=32)[0] >= 16
+    # rows of many sequences: the partials of a partition are large
+    assert decode_split(1024, 30000, 1900, 512, True, rows=32)[0] <= 4
     # whole sequences already fill the CUs many times over
     assert decode_split(4096, 4096, 800, 512, True, rows=8)[0] == 1
 
