@@ -253,7 +253,8 @@ def decode_split(items: int, max_len: int, mean_len: float, item_token_bytes: in
       (measured on lengths within a factor of 30): 128 log-uniform lengths in
       [16, 16384], 64/8 heads 368 -> 291 us, int8 at head_dim 64 182 -> 138,
       four tokens each 372 -> 316; one of 100000 and 63 of 200, 32/1 heads 166
-      -> 67; 2 of 65536 and 30 of 512 88 -> 48; 100 in [100, 10000] 57 -> 47.
+      -> 67; 2 of 65536 and 30 of 512 88 -> 48; 100 in [100, 10000] 57 -> 47; eight tokens each,
+      64 in [16, 65536] 458 -> 420.
     * Eight waves where a CU has one workgroup, but four on the VALU kernels
       for whole sequences below 1024 tokens (240 items of 609 tokens 17.3 ->
       16.8 us, 33 x 8 of 68 11.4 -> 7.8) and in larger grids, except that the
